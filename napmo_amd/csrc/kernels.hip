@@ -7,7 +7,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
-#include "synth_kernel.hpp"
+#include "synth_launch.hpp"
 
 namespace napmo {
 

@@ -5,18 +5,13 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "synth_launch.hpp"
 
 namespace napmo {
 
 // One thread per point, loop over centres. Per (point, centre): one inverse radial
 // transform, then the m-major recurrence of the scaled PI_l^m(z) polynomials of the unit
 // vector (r^2 = 1) and (x + i y)^m, each harmonic contracted with its Horner spline.
-static __device__ inline double rtf_inv(int kind, double p0, double p1, int n, double r) {
-  if (kind == 0) return -(acos((r - p0) / (r + p0)) / p1) + n;
-  if (kind == 1) return pow(r / p0, 1.0 / p1) - 1;
-  return r;
-}
-
 template <int LMAX>
 __global__ void __launch_bounds__(256) k_synth(AtomTables at, const double *__restrict__ px,
                                                const double *__restrict__ py,
