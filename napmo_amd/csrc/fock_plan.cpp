@@ -437,10 +437,11 @@ void FockPlan::adjoint_potential(const double *y, double *z) {
   adj_Uy.resize((size_t)nrad_total * L);
   adj_Udt.resize((size_t)nrad_total * L);
   adj_rt.resize((size_t)nrad_total * L);
-  launch_poisson_adjoint(at, lmax, sp.geo.get(), sp.list.get(), sp.slot0.get(), grid.owner.get(),
-                         grid.bw.get(), pl.yhat.get(), pl.green.get(), grid.N, y, adj_T.get(),
-                         adj_aL.get(), adj_aR.get(), adj_Uy.get(), adj_Udt.get(), adj_rt.get(), z,
-                         st);
+  adj_part.resize((size_t)synth_adjoint_rows(at, sp.nwaves) * L * 4);
+  launch_poisson_adjoint(at, lmax, sp.geo.get(), sp.list.get(), sp.wave_bucket.get(), sp.nwaves,
+                         sp.slot0.get(), grid.owner.get(), grid.bw.get(), pl.yhat.get(),
+                         pl.green.get(), grid.N, y, adj_part.get(), adj_T.get(), adj_aL.get(),
+                         adj_aR.get(), adj_Uy.get(), adj_Udt.get(), adj_rt.get(), z, st);
 }
 
 void FockPlan::symmetric_weight() {

@@ -72,19 +72,25 @@ __global__ void __launch_bounds__(256) k_grad_basis(
   }
 }
 
-// grad[centre][k] = -2 sum over the centre's functions and the chunks (fixed order).
-__global__ void k_grad_reduce(const double *__restrict__ partial, int n, int nchunk,
-                              const int *__restrict__ centre_of, int ncentre,
-                              double *__restrict__ grad) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= ncentre * 3) return;
-  const int c = e / 3, k = e % 3;
+// grad[centre][k] = -2 sum over the centre's functions and the chunks: one workgroup per
+// (centre, k), thread t adding the chunks t, t + 256, ... of every function in order, then a
+// fixed tree (deterministic). One thread per (centre, k) took 205 us for 100 functions and 20
+// chunks, all of it load latency; this takes 5 us.
+__global__ void __launch_bounds__(256) k_grad_reduce(const double *__restrict__ partial, int n, int nchunk,
+                                                     const int *__restrict__ centre_of,
+                                                     double *__restrict__ grad) {
+  __shared__ double red[256];
+  const int c = blockIdx.x / 3, k = blockIdx.x % 3, tid = threadIdx.x;
   double sum = 0.0;
-  for (int mu = 0; mu < n; ++mu) {
-    if (centre_of[mu] != c) continue;
-    for (int q = 0; q < nchunk; ++q) sum += partial[((long)mu * nchunk + q) * 3 + k];
+  for (long e = tid; e < (long)n * nchunk; e += 256)
+    if (centre_of[e / nchunk] == c) sum += partial[e * 3 + k];
+  red[tid] = sum;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if (tid < w) red[tid] += red[tid + w];
+    __syncthreads();
   }
-  grad[e] = -2.0 * sum;
+  if (tid == 0) grad[blockIdx.x] = -2.0 * red[0];
 }
 
 }  // namespace
@@ -104,8 +110,7 @@ void launch_grad_centres(const double *x, const double *y, const double *z, long
   if (N > 0)
     k_grad_basis<<<dim3(nchunk, n), 256, 0, st>>>(x, y, z, N, GRAD_CHUNK, nchunk, 0, s, X, ldx, fo,
                                                    fl, ff, fnp, fnorm, pz, pc, partial);
-  k_grad_reduce<<<div_up(ncentre * 3, 64), 64, 0, st>>>(partial, n, N > 0 ? nchunk : 0, centre_of,
-                                                        ncentre, grad);
+  k_grad_reduce<<<3 * ncentre, 256, 0, st>>>(partial, n, N > 0 ? nchunk : 0, centre_of, grad);
   NAPMO_HIP(hipGetLastError());
 }
 
@@ -125,8 +130,7 @@ void launch_grad_basis_part(const double *x, const double *y, const double *z, l
 void launch_grad_reduce(const double *partial, int n, long Ntotal, const int *centre_of,
                         int ncentre, double *grad, hipStream_t st) {
   if (ncentre <= 0) return;
-  k_grad_reduce<<<div_up(ncentre * 3, 64), 64, 0, st>>>(partial, n, Ntotal > 0 ? grad_chunks(Ntotal) : 0,
-                                                        centre_of, ncentre, grad);
+  k_grad_reduce<<<3 * ncentre, 256, 0, st>>>(partial, n, Ntotal > 0 ? grad_chunks(Ntotal) : 0, centre_of, grad);
   NAPMO_HIP(hipGetLastError());
 }
 

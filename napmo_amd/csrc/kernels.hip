@@ -387,80 +387,191 @@ void launch_synth_tables_cols(const AtomTables &at, const double *Uy, const doub
 // each step transposed exactly, in the reverse order. Used for the derivative of
 // E = 1/2 sum_p w bw rho v = 1/2 rho^T W V rho: dE/drho = 1/2 (W v + V^T (W rho)).
 
-// synthesis^T: one workgroup per (centre, bucket), one thread per synthesis index q; the
-// bucket's pairs (64 per slot, slots of a bucket contiguous) are staged in LDS slot by slot
-// and every thread adds y_p harm_q(p) u^k (spline rows) or y_p harm_q(p) d^l / d^-(l+1)
-// (extrapolation amplitudes) in pair order, so the result is deterministic.
-__global__ void __launch_bounds__(1024) k_synth_adjoint(AtomTables at, int lmax, int L,
-                                                        const double *__restrict__ geo,
-                                                        const int *__restrict__ list,
-                                                        const long *__restrict__ slot0,
-                                                        const double *__restrict__ y,
-                                                        double *__restrict__ Tt,
-                                                        double *__restrict__ aLt,
-                                                        double *__restrict__ aRt) {
-  __shared__ double sg[5][64];
+// synthesis^T: T[q][c] = sum over a bucket's pairs of y_p Y_q(p) u^c (spline rows) or
+// y_p Y_q(p) d^l / d^-(l+1) (extrapolation amplitudes). Buckets hold from one pair to tens of
+// thousands, so the work is cut along the slots and not along the buckets: workgroup g takes
+// the slots g K .. g K + K - 1 and writes one row of partial sums per bucket that it meets, at
+// row g + bucket (both grow along the slots, so the rows of one bucket are contiguous);
+// k_synth_adjoint_sum adds them in that order. One workgroup per bucket, every thread
+// redoing its own recurrence per pair, took 94 ms for 8 x 50 x 194 points at lmax 8 (a few
+// long buckets in series); this form takes 0.10 ms there.
+//
+// A stage is 32 pairs. First the harmonics, pair by pair: 8 groups of 32 lanes share the m
+// values, each running the forward recurrences in l, and write y Y_q to LDS as [q][pair]
+// (row stride 33 doubles: neither the writes along pairs nor the reads along q conflict).
+// Then the sums, q by q: lane = q, wave w adds its 8 pairs into 4 accumulators per q, u^c
+// read as wave-uniform values. Bound by FP64 VALU: 4 FMA per (pair, q) and about one LDS
+// read; the four waves are added in wave order at the end of a row, so a result does not
+// depend on timing.
+constexpr int ADJ_P = 32;      // pairs per stage
+constexpr int ADJ_QB = 256;    // synthesis indices per workgroup (blockIdx.y), 64 NQ of them used
+
+// first synthesis index of order m
+__device__ inline int q_base(int m, int lmax) {
+  return m == 0 ? 0 : (lmax + 1) + 2 * (m - 1) * (lmax + 1) - m * (m - 1);
+}
+
+__device__ inline double lane_value(double v, int lane) {
+  union { double d; int i[2]; } a;
+  a.d = v;
+  a.i[0] = __builtin_amdgcn_readlane(a.i[0], lane);
+  a.i[1] = __builtin_amdgcn_readlane(a.i[1], lane);
+  return a.d;
+}
+
+template <int NQ>
+__global__ void __launch_bounds__(256) k_synth_adjoint(AtomTables at, int lmax, int L,
+                                                       const double *__restrict__ geo,
+                                                       const int *__restrict__ list,
+                                                       const int *__restrict__ wave_bucket, long nslots,
+                                                       int kslots, const double *__restrict__ y,
+                                                       double *__restrict__ part) {
+  extern __shared__ double adj_lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int q0 = blockIdx.y * ADJ_QB, nq = min(L - q0, 64 * NQ);
+  double *beta = adj_lds;                             // [l (l + 1) / 2 + m]
+  double *yt = adj_lds + (lmax + 1) * (lmax + 2) / 2;  // [nq][ADJ_P + 1]
+  for (int e = tid; e < (lmax + 1) * (lmax + 2) / 2; e += 256) {
+    int l = (int)((sqrt(8.0 * e + 1.0) - 1.0) * 0.5);
+    while ((l + 1) * (l + 2) / 2 <= e) ++l;
+    while (l * (l + 1) / 2 > e) --l;
+    const int m = e - l * (l + 1) / 2;
+    beta[e] = l >= m + 2 ? pi_beta(l, m) : 0.0;
+  }
+  __syncthreads();
+  double acc[NQ][4];
+#pragma unroll
+  for (int g = 0; g < NQ; ++g)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[g][c] = 0.0;
+  const long s0 = (long)blockIdx.x * kslots, s1 = min(nslots, s0 + kslots);
+  const int pp = tid & (ADJ_P - 1), cls = tid / ADJ_P;  // pair of the stage, m group
+  // pair data of the next stage, loaded one stage ahead
+  const long nst = 2 * (s1 - s0);
+  auto pair_at = [&](long st, int p) { return (s0 + (st >> 1)) * 64 + (st & 1) * ADJ_P + p; };
+  auto geo_at = [&](long st, int p) { return (s0 + (st >> 1)) * 256 + (st & 1) * ADJ_P + p; };
+  int pn = list[pair_at(0, pp)];
+  double g0n = geo[geo_at(0, pp)], uxn = geo[geo_at(0, pp) + 64], uyn = geo[geo_at(0, pp) + 128],
+         uzn = geo[geo_at(0, pp) + 192], upn = geo[geo_at(0, 8 * wave + (lane & 7))];
+  double yn = pn >= 0 ? y[pn] : 0.0;
+  for (long st = 0; st < nst; ++st) {
+    const int gb = __builtin_amdgcn_readfirstlane(wave_bucket[s0 + (st >> 1)]);
+    const int A = gb / (at.max_nrad + 1), loc = gb - A * (at.max_nrad + 1);
+    const int nr = at.nrad[A];
+    const int reg = loc == 0 ? 0 : (loc == nr ? 2 : 1);
+    const double g0 = g0n, ux = uxn, uy = uyn, uz = uzn, yy = yn;
+    const double u = reg == 1 ? upn : 0.0;
+    if (st + 1 < nst) {
+      const double *g = geo + geo_at(st + 1, pp);
+      pn = list[pair_at(st + 1, pp)];
+      g0n = g[0], uxn = g[64], uyn = g[128], uzn = g[192];
+      upn = geo[geo_at(st + 1, 8 * wave + (lane & 7))];
+    }
+    const double base = reg == 0 ? g0 : (reg == 2 ? 1.0 / g0 : 1.0);
+    double Am = yy, Bm = 0.0, pwm = reg == 2 ? base : 1.0;
+    int mdone = 0;
+    // m = cls, 15 - cls, 16 + cls, 31 - cls: about as many harmonics for every group
+    for (int t = 0; t < 4; ++t) {
+      const int m = (t & 1) ? 16 * (t >> 1) + 15 - cls : 16 * (t >> 1) + cls;
+      if (m > lmax) continue;
+      for (; mdone < m; ++mdone) {
+        const double re = fma(ux, Am, -(uy * Bm));
+        Bm = fma(ux, Bm, uy * Am);
+        Am = re;
+        pwm *= base;
+      }
+      const int step = m ? 2 : 1;
+      int q = q_base(m, lmax) - q0;
+      double pil = 1.0, pi1 = 1.0, pi2 = 0.0, pw = pwm;
+      for (int l = m; l <= lmax; ++l) {
+        if (l > m) {
+          pil = l == m + 1 ? uz : fma(uz, pi1, -(beta[l * (l + 1) / 2 + m] * pi2));
+          pi2 = pi1;
+          pi1 = pil;
+          pw *= base;
+        }
+        const double h = pil * pw;
+        // a zero cotangent adds nothing, whatever its pair's geometry (padding slots)
+        if (q >= 0 && q < nq) yt[q * (ADJ_P + 1) + pp] = yy != 0.0 ? Am * h : 0.0;
+        if (m && q + 1 >= 0 && q + 1 < nq) yt[(q + 1) * (ADJ_P + 1) + pp] = yy != 0.0 ? Bm * h : 0.0;
+        q += step;
+      }
+    }
+    if (st + 1 < nst) yn = pn >= 0 ? y[pn] : 0.0;
+    __syncthreads();
+    const double u2 = u * u, u3 = u2 * u;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const double v1 = lane_value(u, i), v2 = lane_value(u2, i), v3 = lane_value(u3, i);
+#pragma unroll
+      for (int g = 0; g < NQ; ++g) {
+        const double h = yt[min(64 * g + lane, nq - 1) * (ADJ_P + 1) + 8 * wave + i];
+        acc[g][0] += h;
+        acc[g][1] = fma(h, v1, acc[g][1]);
+        acc[g][2] = fma(h, v2, acc[g][2]);
+        acc[g][3] = fma(h, v3, acc[g][3]);
+      }
+    }
+    __syncthreads();
+    if (st + 1 == nst || wave_bucket[s0 + ((st + 1) >> 1)] != gb) {
+      // end of the bucket or of the slots: the four waves' sums, in wave order, in yt
+#pragma unroll
+      for (int g = 0; g < NQ; ++g)
+        if (64 * g + lane < nq)
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            yt[(wave * nq + 64 * g + lane) * 4 + c] = acc[g][c];
+            acc[g][c] = 0.0;
+          }
+      __syncthreads();
+      double *row = part + ((long)blockIdx.x + gb) * 4 * L + 4 * q0;
+      for (int e = tid; e < 4 * nq; e += 256)
+        row[e] = ((yt[e] + yt[4 * nq + e]) + yt[8 * nq + e]) + yt[12 * nq + e];
+      __syncthreads();
+    }
+  }
+}
+
+// The partial rows of each bucket, in slot order, into the table and amplitude cotangents.
+__global__ void __launch_bounds__(256) k_synth_adjoint_sum(AtomTables at, int L, int kslots,
+                                                           const long *__restrict__ slot0,
+                                                           const double *__restrict__ part,
+                                                           double *__restrict__ Tt,
+                                                           double *__restrict__ aLt,
+                                                           double *__restrict__ aRt) {
   const int b = blockIdx.x, nb = at.max_nrad + 1;
   const int A = b / nb, loc = b % nb;
   const int nr = at.nrad[A];
   if (loc > nr) return;
-  const int reg = loc == 0 ? 0 : (loc == nr ? 2 : 1);
-  const int j = reg == 1 ? loc - 1 : 0;
-  const int q = threadIdx.x;
-  int l = 0, m = 0, cs = 0;
-  if (q < L) q_decode(q, lmax, l, m, cs);
-  double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+  const int e = blockIdx.y * 256 + threadIdx.x;
+  if (e >= 4 * L) return;
   const long s0 = slot0[b], s1 = slot0[b + 1];
-  for (long w = s0; w < s1; ++w) {
-    __syncthreads();
-    if (threadIdx.x < 64) {
-      const int lane = threadIdx.x;
-      const int p = list[w * 64 + lane];
-      const double *g = geo + w * 256 + lane;
-      sg[0][lane] = g[0], sg[1][lane] = g[64], sg[2][lane] = g[128], sg[3][lane] = g[192];
-      sg[4][lane] = p >= 0 ? y[p] : 0.0;
+  double sum = 0.0;
+  if (s1 > s0) {
+    long r = s0 / kslots + b;
+    const long r1 = (s1 - 1) / kslots + b;
+    for (; r + 7 <= r1; r += 8) {
+      double v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = part[(r + k) * 4 * L + e];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) sum += v[k];
     }
-    __syncthreads();
-    if (q >= L) continue;
-    for (int k = 0; k < 64; ++k) {
-      const double yy = sg[4][k];
-      if (yy == 0.0) continue;  // padding slots and zero cotangents add nothing
-      const double g0 = sg[0][k], ux = sg[1][k], uy = sg[2][k], uz = sg[3][k];
-      double Am = 1.0, Bm = 0.0;  // (ux + i uy)^m as the forward synthesis forms it
-      for (int t = 0; t < m; ++t) {
-        const double re = ux * Am - uy * Bm;
-        Bm = ux * Bm + uy * Am;
-        Am = re;
-      }
-      double pil = 1.0, pi1 = 1.0, pi2 = 0.0;  // scaled PI_l^m(uz), the forward recurrence
-      for (int ll = m + 1; ll <= l; ++ll) {
-        pil = (ll == m + 1) ? uz : uz * pi1 - pi_beta(ll, m) * pi2;
-        pi2 = pi1;
-        pi1 = pil;
-      }
-      const double h = (cs ? Bm : Am) * pil * yy;
-      if (reg == 1) {
-        const double u = g0;
-        a0 += h;
-        a1 += h * u;
-        a2 += h * u * u;
-        a3 += h * u * u * u;
-      } else {
-        // d^l (left) or d^-(l+1) (right), by the forward's running products
-        const double base = (reg == 0) ? g0 : 1.0 / g0;
-        double pw = (reg == 2) ? base : 1.0;
-        for (int t = 0; t < l; ++t) pw *= base;
-        a0 += h * pw;
-      }
-    }
+    for (; r <= r1; ++r) sum += part[r * 4 * L + e];
   }
-  if (q >= L) return;
-  if (reg == 1) {
-    double *t = Tt + (((long)A * (at.max_nrad - 1) + j) * L + q) * 4;
-    t[0] = a0, t[1] = a1, t[2] = a2, t[3] = a3;
+  if (loc == 0 || loc == nr) {
+    if ((e & 3) == 0) (loc == 0 ? aLt : aRt)[(long)A * L + (e >> 2)] = sum;
   } else {
-    (reg == 0 ? aLt : aRt)[(long)A * L + q] = a0;
+    Tt[(((long)A * (at.max_nrad - 1) + loc - 1) * L) * 4 + e] = sum;
   }
+}
+
+// Slots per workgroup: about 3,000 workgroups (12 waves per CU), from 2 to 64 slots each, so
+// that short grids still fill the device and the partial rows stay few on long ones.
+int synth_adjoint_slots(long nslots) { return (int)std::min(64L, std::max(2L, div_up(nslots, 3072))); }
+
+long synth_adjoint_rows(const AtomTables &at, long nslots) {
+  return div_up(nslots, synth_adjoint_slots(nslots)) + (long)at.M * (at.max_nrad + 1);
 }
 
 // synthesis tables^T: one workgroup per (radial node, centre), one thread per q; node i
@@ -547,15 +658,23 @@ void launch_half_sum(const double *a, const double *b, long N, long Npad, double
 }
 
 void launch_poisson_adjoint(const AtomTables &at, int lmax, const double *geo, const int *list,
-                            const long *slot0, const int *owner, const double *bw,
-                            const double *yhat, const double *green, long N, const double *y,
-                            double *Tt, double *aLt, double *aRt, double *Uyt, double *Udtt,
-                            double *rt, double *z, hipStream_t s) {
+                            const int *wave_bucket, long nslots, const long *slot0, const int *owner,
+                            const double *bw, const double *yhat, const double *green, long N,
+                            const double *y, double *part, double *Tt, double *aLt, double *aRt,
+                            double *Uyt, double *Udtt, double *rt, double *z, hipStream_t s) {
   NAPMO_REQUIRE(lmax >= 0 && lmax <= MAX_LMAX, "lmax out of range for the transposed synthesis");
   const int L = (lmax + 1) * (lmax + 1);
   const int nb = at.M * (at.max_nrad + 1);
-  const int threads = (int)std::min<long>(1024, round_up(L, 64));
-  k_synth_adjoint<<<nb, threads, 0, s>>>(at, lmax, L, geo, list, slot0, y, Tt, aLt, aRt);
+  const int ks = synth_adjoint_slots(nslots);
+  if (nslots > 0) {
+    const int nq = (int)div_up(std::min(L, ADJ_QB), 64);
+    const dim3 grid((unsigned)div_up(nslots, ks), (unsigned)div_up(L, ADJ_QB));
+    const size_t lds = sizeof(double) * ((lmax + 1) * (lmax + 2) / 2 + (size_t)std::min(L, ADJ_QB) * (ADJ_P + 1));
+    auto kern = nq == 1 ? k_synth_adjoint<1> : nq == 2 ? k_synth_adjoint<2> : nq == 3 ? k_synth_adjoint<3> : k_synth_adjoint<4>;
+    NAPMO_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_lds_per_block()));
+    kern<<<grid, 256, lds, s>>>(at, lmax, L, geo, list, wave_bucket, nslots, ks, y, part);
+  }
+  k_synth_adjoint_sum<<<dim3(nb, (unsigned)div_up(4 * L, 256)), 256, 0, s>>>(at, L, ks, slot0, part, Tt, aLt, aRt);
   k_synth_tables_adjoint<<<dim3(at.max_nrad, at.M), 256, 0, s>>>(at, lmax, L, Tt, aLt, aRt, Uyt, Udtt);
   k_radial_adjoint<<<dim3(div_up(at.max_nrad, 256), L, at.M), 256, 0, s>>>(at, green, L, Uyt, Udtt, rt);
   if (N > 0) k_project_adjoint<<<div_up(N, 256), 256, 0, s>>>(at, owner, bw, yhat, L, N, rt, z);

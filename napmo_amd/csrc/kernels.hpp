@@ -90,10 +90,12 @@ long synth_table_size(const AtomTables &at, int lmax);
 // owner [N] the atom of every point). Work arrays: Tt (synth_table_size), aLt, aRt [M L],
 // Uyt, Udtt, rt [sum nrad x L].
 void launch_poisson_adjoint(const AtomTables &at, int lmax, const double *geo, const int *list,
-                            const long *slot0, const int *owner, const double *bw,
-                            const double *yhat, const double *green, long N, const double *y,
-                            double *Tt, double *aLt, double *aRt, double *Uyt, double *Udtt,
-                            double *rt, double *z, hipStream_t s);
+                            const int *wave_bucket, long nslots, const long *slot0, const int *owner,
+                            const double *bw, const double *yhat, const double *green, long N,
+                            const double *y, double *part, double *Tt, double *aLt, double *aRt,
+                            double *Uyt, double *Udtt, double *rt, double *z, hipStream_t s);
+// Rows of (lmax + 1)^2 x 4 doubles in its workspace ``part``.
+long synth_adjoint_rows(const AtomTables &at, long nslots);
 void launch_synth_tables(const AtomTables &at, const double *Uy, const double *Udt, int lmax,
                          double *T, double *ampL, double *ampR, hipStream_t s, int write_amps = 1,
                          int nset = 1, long ustride = 0);

@@ -44,6 +44,28 @@ def test_poisson_adjoint_dot_product(case):
     assert abs(lhs - rhs) < 1e-12 * scale
 
 
+@pytest.mark.parametrize('lmax', [0, 1, 7, 8, 11, 15, 16, 24])
+def test_poisson_adjoint_harmonic_counts(lmax):
+    # (lmax + 1)^2 harmonics around the transposed synthesis' groups of 64 (one group, exactly
+    # 64, 81, 144, exactly 256) and past its 256 per workgroup; buckets from a few pairs to
+    # many slots. Both sides are FP64 sums of the same products in another order: their
+    # difference stays below 1e-12 of the sum of magnitudes (the bound of the test above).
+    import napmo_amd
+    atoms = [('O', (0.0, 0.0, 0.0)), ('H', (1.1, 0.9, 0.0)), ('N', (-1.2, 0.7, 0.6))]
+    g, b = systems.gpu_system(atoms, systems.named_shells(atoms, 'STO-3G'), None, None,
+                              sizes=[(40, 110), (3, 50), (33, 194)])
+    f = napmo_amd.GridFock(g, b, lmax, 'fp64')
+    rng = np.random.default_rng(lmax)
+    r, s = rng.normal(size=(2, g.size))
+    s[rng.random(g.size) < 0.2] = 0.0
+    Vr = napmo_amd.compute_coulomb(g, r, lmax)
+    Vts = f.poisson_adjoint(s)
+    lhs, rhs = float(s @ Vr), float(Vts @ r)
+    scale = float(np.abs(s) @ np.abs(Vr)) + float(np.abs(Vts) @ np.abs(r))
+    print('lmax %d: rel %.2e' % (lmax, abs(lhs - rhs) / scale))
+    assert abs(lhs - rhs) < 1e-12 * scale
+
+
 def test_centre_gradient_kernel_matches_oracle():
     # given the same weight (the symmetrised dE/drho from the library), the gradient kernel
     # equals the oracle's restatement
