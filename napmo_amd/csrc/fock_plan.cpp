@@ -79,7 +79,9 @@ FockPlan::FockPlan(DeviceGrid &g, const BasisSet &b, int lmax_, int prec_mode)
 void FockPlan::reshape() {
   fsh = fock_shape(ld, Npad, true, fock_wg);
   psh = fock_pass_shape(ld, Npad, pass_wg);
-  F_part.resize((size_t)std::max(fsh.nchunk, use_pass ? psh.nchunk : 0) * fsh.cstride());
+  dsh = div_up(n, 16) <= FOCK_MAX_NB ? fock_block_shape(n, ld, Npad, fock_wg) : fsh;
+  const size_t tiles = prec == NAPMO_PREC_BF16X3 ? (size_t)std::max(fsh.nchunk, use_pass ? psh.nchunk : 0) * fsh.cstride() : 0;
+  F_part.resize(std::max(tiles, (size_t)dsh.nchunk * dsh.cstride()));
 }
 
 void FockPlan::set_tuning(int key, long value) {
@@ -158,7 +160,8 @@ void FockPlan::set_tuning(int key, long value) {
 
 long FockPlan::get_tuning(int key) const {
   switch (key) {
-    case NAPMO_TUNE_FOCK_WG: return (long)fsh.nchunk * fsh.ntiles;
+    case NAPMO_TUNE_FOCK_WG:
+      return prec != NAPMO_PREC_BF16X3 && dsh.nb > 0 ? (long)dsh.nchunk * dsh.nstrip : (long)fsh.nchunk * fsh.ntiles;
     case NAPMO_TUNE_PASS_WG: return (long)psh.nchunk;
     case NAPMO_TUNE_USE_PASS: return use_pass;
     case NAPMO_TUNE_DENSITY_KS: return density_ks;
@@ -411,12 +414,12 @@ void FockPlan::contract(int slot, const double *dP, const double *veff, double *
   else if (prec == NAPMO_PREC_BF16X3)
     launch_fock_bf16x3(fsh, phiT_hi.get(), phiT_lo.get(), phiT32.get(), s.get(), F_part.get(), st);
   else
-    launch_fock_f64(fsh, phi64.get(), phi64.get(), s.get(), F_part.get(), st);
+    launch_fock_f64(dsh, phi64.get(), phi64.get(), s.get(), F_part.get(), st);
   mark(slot, 8);
   if (use_pass)
     launch_fock_reduce_f32(psh, part32, n, dF, st);
   else
-    launch_fock_reduce(fsh, F_part.get(), n, 0, 1.0, 0, dF, st);
+    launch_fock_reduce(prec == NAPMO_PREC_BF16X3 ? fsh : dsh, F_part.get(), n, 0, 1.0, 0, dF, st);
   mark(slot, 9);
   launch_traces(dP, dF, n, grid.wbw.get(), rho.get(), veff, grid.N, dE, trace_work.get(), st);
   mark(slot, 10);
@@ -460,7 +463,7 @@ void FockPlan::symmetric_weight() {
 // gradient's 4096-point chunk and of the density tile, so every partial sum covers the same
 // points as in the stored-Phi path.
 long FockPlan::backward_chunk() const {
-  const long unit = std::lcm(std::lcm(fsh.chunk, grad_chunk_points()), 256L);
+  const long unit = std::lcm(std::lcm(dsh.chunk, grad_chunk_points()), 256L);
   return std::max<long>(1, div_up(std::max<long>(bwd_points, 1), unit)) * unit;
 }
 
@@ -468,7 +471,7 @@ void FockPlan::energy_dP(double *dEdP) {
   symmetric_weight();
   hipStream_t st = stream;
   if (bwd_points <= 0) {
-    launch_fock_f64(fsh, phi64.get(), phi64.get(), ssym.get(), F_part.get(), st);
+    launch_fock_f64(dsh, phi64.get(), phi64.get(), ssym.get(), F_part.get(), st);
   } else {
     // Phi recollocated chunk by chunk; each chunk's Fock partials land where the stored-Phi
     // launch writes them
@@ -478,14 +481,14 @@ void FockPlan::energy_dP(double *dEdP) {
       const long cn = std::max<long>(0, std::min(C, grid.N - p0)), cpad = std::min(C, Npad - p0);
       basis.collocate(grid.x.get() + p0, grid.y.get() + p0, grid.z.get() + p0, cn, cpad, ld,
                       bwd_phi.get(), nullptr, st);
-      FockShape cs = fsh;
+      FockShape cs = dsh;
       cs.Npad = cpad;
-      cs.nchunk = (int)div_up(cpad, fsh.chunk);
+      cs.nchunk = (int)div_up(cpad, dsh.chunk);
       launch_fock_f64(cs, bwd_phi.get(), bwd_phi.get(), ssym.get() + p0,
-                      F_part.get() + (p0 / fsh.chunk) * fsh.cstride(), st);
+                      F_part.get() + (p0 / dsh.chunk) * dsh.cstride(), st);
     }
   }
-  launch_fock_reduce(fsh, F_part.get(), n, 0, 1.0, 0, dEdP, st);
+  launch_fock_reduce(dsh, F_part.get(), n, 0, 1.0, 0, dEdP, st);
 }
 
 void FockPlan::gradient_device(const double *dP, double *dG) {
@@ -596,11 +599,11 @@ void FockPlan::contract_potential(const double *v_host, double *F_out) {
   else if (prec == NAPMO_PREC_BF16X3)
     launch_fock_bf16x3(fsh, phiT_hi.get(), phiT_lo.get(), phiT32.get(), s.get(), F_part.get(), st);
   else
-    launch_fock_f64(fsh, phi64.get(), phi64.get(), s.get(), F_part.get(), st);
+    launch_fock_f64(dsh, phi64.get(), phi64.get(), s.get(), F_part.get(), st);
   if (use_pass)
     launch_fock_reduce_f32(psh, part32, n, F.get(), st);
   else
-    launch_fock_reduce(fsh, F_part.get(), n, 0, 1.0, 0, F.get(), st);
+    launch_fock_reduce(prec == NAPMO_PREC_BF16X3 ? fsh : dsh, F_part.get(), n, 0, 1.0, 0, F.get(), st);
   F.download(F_out, (size_t)n * n, st);
   NAPMO_HIP(hipStreamSynchronize(st));
 }
@@ -608,8 +611,8 @@ void FockPlan::contract_potential(const double *v_host, double *F_out) {
 void FockPlan::overlap(double *S_out) {
   hipStream_t st = stream;
   launch_scale3(grid.w.get(), grid.bw.get(), nullptr, grid.N, Npad, s.get(), st);
-  launch_fock_f64(fsh, phi64.get(), phi64.get(), s.get(), F_part.get(), st);
-  launch_fock_reduce(fsh, F_part.get(), n, 0, 1.0, 0, F.get(), st);
+  launch_fock_f64(dsh, phi64.get(), phi64.get(), s.get(), F_part.get(), st);
+  launch_fock_reduce(dsh, F_part.get(), n, 0, 1.0, 0, F.get(), st);
   F.download(S_out, (size_t)n * n, st);
   NAPMO_HIP(hipStreamSynchronize(st));
 }

@@ -148,7 +148,7 @@ GroupPlan::GroupPlan(const std::vector<FockPlan *> &ps, const std::vector<double
   std::vector<DensityMember> dm(nm);
   std::vector<RhoReduceMember> rm(nm);
   std::vector<ScaleMember> sm(nm);
-  std::vector<FockMember> fm(nm);
+  std::vector<FockMember> fm[2];
   for (int m = 0; m < nm; ++m) {
     FockPlan &q = *plans[m];
     const long N = q.grid.N;
@@ -158,12 +158,20 @@ GroupPlan::GroupPlan(const std::vector<FockPlan *> &ps, const std::vector<double
     rho_blocks += div_up(N, 256);
     sm[m] = ScaleMember{q.s.get(), p0[m], N, q.Npad, scale_blocks, A0[m], A0[m + 1]};
     scale_blocks += div_up(q.Npad, 256);
-    fock_blocks += fock_group_fill(fm[m], q.fsh, q.phi64.get(), q.s.get(), q.F_part.get(), fock_blocks);
+    const int w = fock_group_waves(q.dsh) == 8;
+    FockMember f;
+    const long nbl = fock_group_fill(f, q.dsh, q.phi64.get(), q.s.get(), q.F_part.get(), fock[w].blocks);
+    fm[w].push_back(f);
+    fock[w].blocks += nbl;
+    fock[w].lds = std::max(fock[w].lds, fock_group_lds(q.dsh));
   }
   dmem.upload(dm, stream);
   rmem.upload(rm, stream);
   smem.upload(sm, stream);
-  fmem.upload(fm, stream);
+  for (int w = 0; w < 2; ++w) {
+    fock[w].count = (int)fm[w].size();
+    fock[w].mem.upload(fm[w], stream);
+  }
   if (coupled) {
     std::vector<SpeciesSum> ss(nm);
     for (int m = 0; m < nm; ++m) ss[m] = SpeciesSum{A0[m], A0[m + 1], charge[m]};
@@ -197,7 +205,7 @@ void GroupPlan::io_tables(IoTables &io, const double *const *dP, double *const *
     NAPMO_REQUIRE(dP[m] && dF[m] && dE[m], "group build: null pointer");
     pm[m] = PadMember{dP[m], q.P.get(), pad_blocks, q.n, q.n, q.ld, q.ld};
     pad_blocks += div_up((long)q.ld * q.ld, 256);
-    fred_blocks += fock_reduce_group_fill(frm[m], q.fsh, q.F_part.get(), q.n, dF[m], fred_blocks);
+    fred_blocks += fock_reduce_group_fill(frm[m], q.dsh, q.F_part.get(), q.n, dF[m], fred_blocks);
     const double *vs = coupled ? veff.get() : v.get();
     tm[m] = TraceMember{dP[m], dF[m], ug.wbw.get() + p0[m], rho.get() + p0[m], vs + p0[m],
                         dE[m], q.trace_work.get(), (long)q.n * q.n, q.grid.N};
@@ -250,7 +258,8 @@ void GroupPlan::launches(const IoTables &io) {
   else
     launch_contrib_reduce_scale_group(smem.get(), nm, scale_blocks, pairs.contrib.get(), cbase.get(),
                                       ug.wbw.get(), v.get(), stream);
-  launch_fock_group(fmem.get(), nm, fock_blocks, stream);
+  for (int w = 0; w < 2; ++w)
+    launch_fock_group(fock[w].mem.get(), fock[w].count, fock[w].blocks, w ? 8 : 4, fock[w].lds, stream);
   launch_fock_reduce_group(io.frmem.get(), nm, io.fred_blocks, stream);
   launch_traces_group(io.tmem.get(), nm, stream);
   if (coupled) {

@@ -36,8 +36,15 @@ struct GroupPlan {
   DeviceBuffer<DensityMember> dmem;
   DeviceBuffer<RhoReduceMember> rmem;
   DeviceBuffer<ScaleMember> smem;
-  DeviceBuffer<FockMember> fmem;
-  long dens_blocks = 0, rho_blocks = 0, scale_blocks = 0, fock_blocks = 0;
+  long dens_blocks = 0, rho_blocks = 0, scale_blocks = 0;
+  // Fock contraction: one launch for the members with 4 waves per workgroup, one for those
+  // with 8 (more than 320 functions)
+  struct FockGroup {
+    DeviceBuffer<FockMember> mem;
+    int count = 0;
+    long blocks = 0;
+    size_t lds = 0;
+  } fock[2];
   // tables that name the build's inputs and outputs: one set for eager builds, one for
   // the captured graph (which reads its tables at every replay, so eager builds on other
   // pointers must not rewrite them)

@@ -1119,7 +1119,6 @@ void launch_axpby(double a, const double *x, double b, const double *y, long N, 
 //   A[16 x 4]:  lane i holds A[i % 16][i / 16]
 //   B[4 x 16]:  lane i holds B[i / 16][i % 16]
 //   D[16 x 16]: lane i holds D[(i / 16) + 4 r][i % 16] in accumulator element r = 0..3
-constexpr int KS = 16;  // K elements staged in LDS per step (FP64 Fock kernel)
 
 __global__ void k_rho_reduce(const double *__restrict__ partial, int nt, long Npad, long N,
                              double scale, double *__restrict__ rho) {
@@ -1163,266 +1162,6 @@ __global__ void k_scale3(const double *__restrict__ a, const double *__restrict_
 void launch_scale3(const double *a, const double *b, const double *c, long N, long Npad, double *s,
                    hipStream_t st) {
   k_scale3<<<div_up(Npad, 256), 256, 0, st>>>(a, b, c, N, Npad, s);
-  NAPMO_HIP(hipGetLastError());
-}
-
-// =================================================== contractions: FP64 MFMA Fock
-// F[mu][nu] = sum_p X[p][mu] s[p] Y[p][nu]: A[m][k] = X[p0+k][mu0+m], B[k][n] =
-// s[p0+k] Y[p0+k][nu0+n]. Split over points (chunks); one workgroup per (tile, chunk).
-FockShape fock_shape(int ld, long Npad, bool symmetric, long wg_target) {
-  FockShape sh;
-  sh.ld = ld;
-  sh.nt = ld / TILE;
-  sh.ntiles = symmetric ? sh.nt * (sh.nt + 1) / 2 : sh.nt * sh.nt;
-  sh.symmetric = symmetric;
-  sh.Npad = Npad;
-  // aim at ~2048 workgroups (or wg_target); chunks a multiple of 256 points (the mixed
-  // kernel's FP32 accumulation block)
-  long want = std::max(1L, (wg_target > 0 ? wg_target : 2048L) / sh.ntiles);
-  long chunk = round_up(div_up(Npad, want), 256);
-  sh.chunk = std::max<long>(chunk, 256);
-  sh.nchunk = (int)div_up(Npad, sh.chunk);
-  return sh;
-}
-
-__device__ inline void tile_coords(int t, int nt, bool symmetric, int &ti, int &tj) {
-  if (!symmetric) {
-    ti = t / nt, tj = t % nt;
-    return;
-  }
-  int i = 0, rem = t;
-  while (rem >= nt - i) rem -= nt - i, ++i;
-  ti = i, tj = i + rem;
-}
-
-// Points run in stages of KS: the next stage's rows (4 consecutive doubles of one point
-// per thread for each operand) are loaded into registers while the current stage's MFMAs
-// run, then stored to the other LDS buffer (one barrier per stage). LDS rows hold 64
-// functions plus 16 doubles of padding, so a 16 x 4 fragment read touches each bank once
-// per half-wave.
-constexpr int FSTRIDE = TILE + 16;
-
-__device__ __forceinline__ void fock_f64_body(const double *__restrict__ X,
-                                              const double *__restrict__ Yv,
-                                              const double *__restrict__ s, int ld, int nt,
-                                              int symmetric, int ntiles, int nchunk, long Npad,
-                                              long chunk, double *__restrict__ partial, int g) {
-  __shared__ double As[2][KS][FSTRIDE];  // As[.][k][m] = X[p0 + k][mu0 + m]
-  __shared__ double Bs[2][KS][FSTRIDE];  // Bs[.][k][n] = s[p0 + k] Y[p0 + k][nu0 + n]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // XCD-aware order: workgroup g runs on XCD g % 8; all tiles of one chunk of points get
-  // ids congruent mod 8 (g = 8 i + x: tile i % ntiles, chunk (i / ntiles) * 8 + x), so the
-  // chunk's Phi rows are shared through one L2
-  const int xcd = g & 7, gi = g >> 3;
-  const int tile = gi % ntiles, chunk_id = (gi / ntiles) * 8 + xcd;
-  if (chunk_id >= nchunk) return;
-  int ti, tj;
-  tile_coords(tile, nt, symmetric, ti, tj);
-  const int mu0 = ti * TILE, nu0 = tj * TILE;
-  const bool same = (X == Yv) && (ti == tj);
-  const long pbeg = (long)chunk_id * chunk;
-  const long pend = min(Npad, pbeg + chunk);
-  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
-  const int lr = tid >> 4, lc = (tid & 15) * 4;  // this thread's stage row and 4 columns
-  d4 ra, rb;
-  double rs = 0.0;
-  auto load = [&](long k0) {
-    const long p = k0 + lr;
-    ra = *(const d4 *)&X[p * ld + mu0 + lc];
-    if (!same) rb = *(const d4 *)&Yv[p * ld + nu0 + lc];
-    rs = s[p];
-  };
-  auto store = [&](int buf) {
-    const d4 b = same ? ra : rb;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      As[buf][lr][lc + e] = ra[e];
-      Bs[buf][lr][lc + e] = rs * b[e];
-    }
-  };
-  d4 acc[2][2];
-  for (int a = 0; a < 2; ++a)
-    for (int b = 0; b < 2; ++b) acc[a][b] = (d4){0, 0, 0, 0};
-  if (pbeg < pend) {
-    load(pbeg);
-    store(0);
-  }
-  __syncthreads();
-  int buf = 0;
-  const int kr0 = lane >> 4, mi = lane & 15;
-  for (long k0 = pbeg; k0 < pend; k0 += KS) {
-    const bool more = k0 + KS < pend;
-    if (more) load(k0 + KS);
-#pragma unroll
-    for (int ks = 0; ks < KS; ks += 4) {
-      const int kr = ks + kr0;
-      const double a0 = As[buf][kr][wr + mi], a1 = As[buf][kr][wr + 16 + mi];
-      const double b0 = Bs[buf][kr][wc + mi], b1 = Bs[buf][kr][wc + 16 + mi];
-      acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
-      acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[0][1], 0, 0, 0);
-      acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
-      acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
-    }
-    if (more) store(buf ^ 1);
-    __syncthreads();
-    buf ^= 1;
-  }
-  double *out = partial + (long)chunk_id * ((long)ntiles * TILE * TILE + 32) +
-                (long)tile * TILE * TILE;
-  const int col16 = lane & 15, rg = lane >> 4;
-  for (int a = 0; a < 2; ++a)
-    for (int b = 0; b < 2; ++b)
-      for (int r = 0; r < 4; ++r)
-        out[(wr + a * 16 + rg + 4 * r) * TILE + wc + b * 16 + col16] = acc[a][b][r];
-}
-
-__global__ void __launch_bounds__(256) k_fock_f64(const double *__restrict__ X,
-                                                  const double *__restrict__ Yv,
-                                                  const double *__restrict__ s, int ld, int nt,
-                                                  int symmetric, int ntiles, int nchunk, long Npad,
-                                                  long chunk, double *__restrict__ partial) {
-  fock_f64_body(X, Yv, s, ld, nt, symmetric, ntiles, nchunk, Npad, chunk, partial, blockIdx.x);
-}
-
-// symmetric F = Phi^T diag(s) Phi of many plans in one launch
-__global__ void __launch_bounds__(256) k_fock_f64_group(const FockMember *__restrict__ mem, int nmem) {
-  const long g = blockIdx.x;
-  const FockMember &f = mem[group_member(mem, nmem, g)];
-  fock_f64_body(f.X, f.X, f.s, f.ld, f.nt, 1, f.ntiles, f.nchunk, f.Npad, f.chunk, f.partial,
-                (int)(g - f.block0));
-}
-
-long fock_group_fill(FockMember &f, const FockShape &sh, const double *X, const double *s,
-                     double *partial, long block0) {
-  NAPMO_REQUIRE(sh.symmetric && block0 % 8 == 0, "grouped Fock: symmetric shapes, aligned blocks");
-  f.X = X, f.s = s, f.partial = partial, f.Npad = sh.Npad, f.chunk = sh.chunk, f.block0 = block0;
-  f.ld = sh.ld, f.nt = sh.nt, f.ntiles = sh.ntiles, f.nchunk = sh.nchunk;
-  return (long)sh.ntiles * round_up(sh.nchunk, 8);
-}
-
-void launch_fock_group(const FockMember *d_mem, int nmem, long nblocks, hipStream_t st) {
-  if (nmem <= 0 || nblocks <= 0) return;
-  k_fock_f64_group<<<dim3((unsigned)nblocks), 256, 0, st>>>(d_mem, nmem);
-  NAPMO_HIP(hipGetLastError());
-}
-
-void launch_fock_f64(const FockShape &sh, const double *X, const double *Y, const double *s,
-                     double *partial, hipStream_t st) {
-  const dim3 grid((unsigned)(sh.ntiles * round_up(sh.nchunk, 8)));
-  k_fock_f64<<<grid, 256, 0, st>>>(X, Y, s, sh.ld, sh.nt, sh.symmetric ? 1 : 0, sh.ntiles,
-                                   sh.nchunk, sh.Npad, sh.chunk, partial);
-  NAPMO_HIP(hipGetLastError());
-}
-
-// Sum the chunk partials of each computed tile element: 4 slices of chunks per element
-// (slice k takes chunks k, k + 4, ...), combined in slice order (deterministic). Threads
-// walk the tile-element space of the partials, so every load is coalesced; the mirror
-// image of an off-diagonal upper tile is written by the same thread. Partials are FP64
-// (per-tile kernels) or FP32 (the one-pass mixed kernel, whose accumulators are FP32).
-template <class T>
-__device__ __forceinline__ void fock_reduce_body(const T *__restrict__ partial, int nt, int ntiles,
-                                                 int nchunk, int symmetric, int n,
-                                                 int upper_mirror, double scale, int accumulate,
-                                                 double *__restrict__ F, long g) {
-  __shared__ double red[4][64];
-  const int el = threadIdx.x & 63, slice = threadIdx.x >> 6;
-  const long u = g * 64 + el;
-  const long nel = (long)ntiles * TILE * TILE;
-  double sum = 0.0;
-  if (u < nel) {
-    const long cstride = nel + 32;
-    int c = slice;
-    // 8 loads in flight, added in chunk order
-    for (; c + 28 < nchunk; c += 32) {
-      double v[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) v[k] = (double)partial[(long)(c + 4 * k) * cstride + u];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) sum += v[k];
-    }
-    for (; c < nchunk; c += 4) sum += (double)partial[(long)c * cstride + u];
-  }
-  red[slice][el] = sum;
-  __syncthreads();
-  if (slice != 0 || u >= nel) return;
-  const double tot = ((red[0][el] + red[1][el]) + red[2][el] + red[3][el]) * scale;
-  const int t = (int)(u / (TILE * TILE)), r = (int)(u % (TILE * TILE)) / TILE, cc = (int)(u % TILE);
-  int ti, tj;
-  if (symmetric) {
-    // upper tiles in row order: (0,0), (0,1), ..., (0,nt-1), (1,1), ...
-    int rem = t;
-    ti = 0;
-    while (rem >= nt - ti) rem -= nt - ti, ++ti;
-    tj = ti + rem;
-  } else {
-    ti = t / nt, tj = t % nt;
-  }
-  const int i = ti * TILE + r, j = tj * TILE + cc;
-  if (i >= n || j >= n) return;
-  auto put = [&](int a, int b) {
-    const long e = (long)a * n + b;
-    F[e] = accumulate ? F[e] + tot : tot;
-  };
-  if (symmetric) {
-    // the upper triangle is mirrored, so F is exactly symmetric (a diagonal tile's own
-    // lower half, equal to rounding, is not used)
-    if (i > j) return;
-    put(i, j);
-    if (i != j) put(j, i);
-  } else if (upper_mirror) {
-    if (i <= j) {
-      put(i, j);
-      if (i != j) put(j, i);
-    }
-  } else {
-    put(i, j);
-  }
-}
-
-template <class T>
-__global__ void __launch_bounds__(256) k_fock_reduce(const T *__restrict__ partial, int nt,
-                                                     int ntiles, int nchunk, int symmetric, int n,
-                                                     int upper_mirror, double scale, int accumulate,
-                                                     double *__restrict__ F) {
-  fock_reduce_body<T>(partial, nt, ntiles, nchunk, symmetric, n, upper_mirror, scale, accumulate,
-                      F, blockIdx.x);
-}
-
-__global__ void __launch_bounds__(256) k_fock_reduce_group(const FockReduceMember *__restrict__ mem,
-                                                           int nmem) {
-  const long g = blockIdx.x;
-  const FockReduceMember &f = mem[group_member(mem, nmem, g)];
-  fock_reduce_body<double>(f.partial, f.nt, f.ntiles, f.nchunk, 1, f.n, 0, 1.0, 0, f.F, g - f.block0);
-}
-
-long fock_reduce_group_fill(FockReduceMember &f, const FockShape &sh, const double *partial, int n,
-                            double *F, long block0) {
-  NAPMO_REQUIRE(sh.symmetric, "grouped Fock reduction: symmetric shapes");
-  f.partial = partial, f.F = F, f.block0 = block0;
-  f.nt = sh.nt, f.ntiles = sh.ntiles, f.nchunk = sh.nchunk, f.n = n;
-  return div_up((long)sh.ntiles * TILE * TILE, 64);
-}
-
-void launch_fock_reduce_group(const FockReduceMember *d_mem, int nmem, long nblocks, hipStream_t st) {
-  if (nmem <= 0 || nblocks <= 0) return;
-  k_fock_reduce_group<<<dim3((unsigned)nblocks), 256, 0, st>>>(d_mem, nmem);
-  NAPMO_HIP(hipGetLastError());
-}
-
-void launch_fock_reduce(const FockShape &sh, const double *partial, int n, int upper_mirror,
-                        double scale, int accumulate, double *F, hipStream_t st) {
-  const long nel = (long)sh.ntiles * TILE * TILE;
-  k_fock_reduce<double><<<div_up(nel, 64), 256, 0, st>>>(partial, sh.nt, sh.ntiles, sh.nchunk,
-                                                         sh.symmetric ? 1 : 0, n, upper_mirror,
-                                                         scale, accumulate, F);
-  NAPMO_HIP(hipGetLastError());
-}
-
-void launch_fock_reduce_f32(const FockShape &sh, const float *partial, int n, double *F,
-                            hipStream_t st) {
-  const long nel = (long)sh.ntiles * TILE * TILE;
-  k_fock_reduce<float><<<div_up(nel, 64), 256, 0, st>>>(partial, sh.nt, sh.ntiles, sh.nchunk,
-                                                        sh.symmetric ? 1 : 0, n, 0, 1.0, 0, F);
   NAPMO_HIP(hipGetLastError());
 }
 

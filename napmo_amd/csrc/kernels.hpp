@@ -244,15 +244,22 @@ void launch_scale3(const double *a, const double *b, const double *c, long N, lo
 
 // F = X^T diag(s) Y over Npad points. symmetric: only upper tiles of F (X == Y).
 // partial buffer: [nchunk x ntiles x TILE x TILE]. Returns nothing; F written by reduce.
+// nb > 0: the upper 16 x 16 blocks instead of 64 x 64 tiles (fock_block_shape, FP64 symmetric
+// contractions only), partial buffer [nchunk x nb (nb + 1) / 2 x 256].
 struct FockShape {
   int ld, nt, ntiles, nchunk;
   long Npad, chunk;
   bool symmetric;
-  // doubles between consecutive chunks' partials: ntiles * TILE * TILE plus 256 B, so the
-  // chunks of one element do not all fall on the same few L2 channels
-  long cstride() const { return (long)ntiles * TILE * TILE + 32; }
+  int nb = 0, bpw = 0, nstrip = 0, nset = 0;  // block rows, blocks per wave, strips, point sets
+  // doubles between consecutive chunks' partials: their elements plus 256 B, so the chunks of
+  // one element do not all fall on the same few L2 channels
+  long cstride() const {
+    return (nb > 0 ? (long)nb * (nb + 1) / 2 * 256 : (long)ntiles * TILE * TILE) + 32;
+  }
 };
 FockShape fock_shape(int ld, long Npad, bool symmetric, long wg_target = 0);
+constexpr int FOCK_MAX_NB = 40;  // most block rows of the block shape (n <= 640)
+FockShape fock_block_shape(int n, int ld, long Npad, long wg_target = 0);
 void launch_fock_f64(const FockShape &sh, const double *X, const double *Y, const double *s,
                      double *partial, hipStream_t st);
 // F_out [n x n] row-major from the partials; symmetric mirrors upper tiles;
@@ -361,14 +368,14 @@ struct DensityMember {   // P-form density of one plan
 struct FockMember {      // FP64 Fock partials of one plan
   const double *X, *s;
   double *partial;
-  long Npad, chunk, block0;
-  int ld, nt, ntiles, nchunk;
+  long Npad, chunk, block0, cstride;
+  int ld, nt, ntiles, nchunk, nb, bpw, nstrip, nset;
 };
 struct FockReduceMember {
   const double *partial;
   double *F;
-  long block0;
-  int nt, ntiles, nchunk, n;
+  long block0, cstride;
+  int nt, ntiles, nchunk, n, nb;
 };
 struct TraceMember {     // E[0] = 1/2 sum P o F, E[1] = 1/2 sum wbw rho v
   const double *P, *F, *wbw, *rho, *v;
@@ -412,7 +419,11 @@ void launch_density_group(const DensityMember *d_mem, int nmem, long nblocks, in
                           hipStream_t s);
 long fock_group_fill(FockMember &f, const FockShape &sh, const double *X, const double *s,
                      double *partial, long block0);
-void launch_fock_group(const FockMember *d_mem, int nmem, long nblocks, hipStream_t st);
+// waves (4 or 8) and LDS of one member's workgroups: a launch takes members of one wave count,
+// with the largest LDS among them
+int fock_group_waves(const FockShape &sh);
+size_t fock_group_lds(const FockShape &sh);
+void launch_fock_group(const FockMember *d_mem, int nmem, long nblocks, int waves, size_t lds, hipStream_t st);
 long fock_reduce_group_fill(FockReduceMember &f, const FockShape &sh, const double *partial, int n,
                             double *F, long block0);
 void launch_fock_reduce_group(const FockReduceMember *d_mem, int nmem, long nblocks, hipStream_t st);
