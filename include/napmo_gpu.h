@@ -434,8 +434,8 @@ enum {
   NAPMO_TUNE_PASS_WG = 1,  /* workgroups of the one-pass BF16x3 Fock kernel; 0 = default */
   NAPMO_TUNE_USE_PASS = 2, /* 0: per-tile BF16x3 kernel, 1: one-pass BF16x3 kernel,
                               2: one-pass kernel on G = sqrt|s| Phi (F = G^T diag(sign s) G) */
-  NAPMO_TUNE_DENSITY_KS = 3, /* K per LDS stage of the density kernels: 16 or 32; 0 = 16 */
-  NAPMO_TUNE_DENSITY_PF = 4, /* stages in flight in the density kernels: 1 or 2; 0 = 1 */
+  NAPMO_TUNE_DENSITY_KS = 3, /* 16 or 32, 0 = 16: accepted and kept, no kernel uses it now */
+  NAPMO_TUNE_DENSITY_PF = 4, /* 1 or 2, 0 = 1: accepted and kept, no kernel uses it now */
   NAPMO_TUNE_SYNTH_NP = 5,   /* (point, centre) pairs per lane of the synthesis, 1 or 2; 0 = 2
                                 (a property of the grid: shared by every plan on it) */
   NAPMO_TUNE_DENSITY_STREAM = 6, /* orbital-form density: 1..4 keep C in LDS and stream Phi when

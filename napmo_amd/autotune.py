@@ -3,8 +3,7 @@
 For a plan (one molecule's grid, basis and precision) it times every candidate launch
 shape of the Fock contraction on the device (the per-tile FP64 / BF16x3 kernels' workgroup
 count, the one-pass BF16x3 kernel's workgroup count, and the choice between the two
-BF16x3 kernels) together with the K depth and prefetch depth of the density kernels' LDS
-stages, then the synthesis' pairs per lane (1 or 2) together with the orbital-form density's
+BF16x3 kernels), then the synthesis' pairs per lane (1 or 2) together with the orbital-form density's
 choice of kernel (C resident in LDS with Phi streamed in one of two launch shapes, or the
 LDS-staged kernel), keeps the fastest, and stores it in a JSON cache keyed by the shape class
 (precision, padded basis size, point count rounded to a power of two), so later plans of
@@ -43,7 +42,7 @@ def shape_key(fock):
 
 
 def candidates(fock):
-    """Launch shapes of the Fock contraction, each with both density stage depths."""
+    """Launch shapes of the Fock contraction."""
     if fock.precision == 'int8':
         # points per chunk (about N / 128 .. N / 512 chunks; every chunk is one workgroup per
         # row group and one FP64 partial of F; with screening, shorter chunks keep fewer
@@ -61,10 +60,7 @@ def candidates(fock):
         out += [{'use_pass': 0, 'fock_wg': w} for w in (1024, 2048, 4096)]
     else:
         out = [{'fock_wg': w} for w in (512, 1024, 2048, 4096, 8192)]
-    ks = [16, 32] if (-(-fock.nbasis // 64) * 64) % 32 == 0 else [16]
-    if fock.precision == 'int8':   # the orbital-form density's knobs are tuned in the second stage
-        return out
-    return [dict(c, density_ks=k, density_pf=f) for c in out for k in ks for f in (1, 2)]
+    return out
 
 
 def apply(fock, setting):

@@ -1,15 +1,11 @@
-// Grid density on FP64 MFMA: X = Phi B over a tile of points, then one of two epilogues.
-//   P form       (B = P [ld x ld]):     rho_partial[ct][p] = sum_{c in tile ct} X_pc Phi_pc
-//   orbital form (B = C [ld x ldc]):    rho_partial[ct][p] = sum_{c in tile ct} X_pc^2
-//   product      (B [ld x ldb]):        X [Npad x ldb] itself (the gradient's Phi P)
+// Grid density on FP64 MFMA: X = Phi B, then rho from X
 // (napmo/wavefunction/psi_hybrid.py:144-154 and napmo/wavefunction/psi_numeric.py:361-369).
-//
-// Workgroup: 128 points x 16 NB columns, 4 waves; wave w owns points 32 w .. 32 w + 31
-// (two 16-row blocks) and all NB column blocks. K runs in stages of DKS (16 or 32): the next stage's
-// Phi rows and B rows are loaded into registers while the MFMAs of the current stage run,
-// then stored to the other LDS buffer (one barrier per stage). LDS rows are padded so each
-// 16 x 4 fragment read of a wave touches every bank once per half.
+//   P form:       rho_p = sum_c X_pc Phi_pc with B the fold of P onto its lower block triangle
+//   orbital form: rho_p = sum_c X_pc^2 with B = C (k_density_tiles; k_density_orb_stream when C
+//                 fits in LDS)
+//   product:      X [Npad x ldb] itself (the gradient's Phi P; k_phi_times)
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -28,12 +24,6 @@ typedef double d2 __attribute__((ext_vector_type(2)));
 
 namespace {
 
-constexpr int DPT = 128;        // points per workgroup
-constexpr int ASTRIDE = DPT + 16;
-constexpr int MODE_P = 0, MODE_ORB = 1, MODE_STORE_X = 2;
-
-constexpr int bstride(int nb) { return (16 * nb) % 32 == 16 ? 16 * nb : 16 * nb + 16; }
-
 // Workgroup g runs on XCD g % 8 (round-robin dispatch); the column tiles of one point
 // tile are given ids that are congruent mod 8, so they share that XCD's L2 and the point
 // tile's Phi rows come from HBM once: g = 8 i + x, column tile i % nct, point tile
@@ -45,151 +35,263 @@ __device__ inline bool xcd_tile(int g, int nct, int npt, int &pt, int &ct) {
   return pt < npt;
 }
 
-// The kernel body for workgroup g (blockIdx.x, or the local index of a grouped launch).
-template <int NB, int MODE, int DKS, int PF>
-__device__ __forceinline__ void density_mfma_body(const double *__restrict__ phi, int ld,
-                                                  long Npad, const double *__restrict__ B,
-                                                  int ldb, int kend, double scale, long nvalid,
-                                                  double *__restrict__ partial, int g) {
-  constexpr int BS = bstride(NB);
+// ------------------------------------------------------------------------ product X = Phi B
+// Workgroup: 128 points x 64 columns, 4 waves; wave w owns points 32 w .. 32 w + 31 and all 64
+// columns. K runs in stages of 16: the next stage's Phi rows and B rows are loaded into
+// registers while the MFMAs of the current stage run, then stored to the other LDS buffer. LDS
+// rows are padded so each 16 x 4 fragment read of a wave touches every bank once per half.
+constexpr int DPT = 128, DKS = 16;
+constexpr int ASTRIDE = DPT + 16, BSTRIDE = TILE + 16;
+
+__global__ void __launch_bounds__(256) k_phi_times(const double *__restrict__ phi, int ld, long Npad,
+                                                   const double *__restrict__ B, int ldb,
+                                                   double *__restrict__ X) {
   __shared__ double As[2][DKS][ASTRIDE];  // As[.][k][m] = Phi[p0 + m][k0 + k]
-  __shared__ double Bs[2][DKS][BS];       // Bs[.][k][c] = B[k0 + k][c0 + c]
+  __shared__ double Bs[2][DKS][BSTRIDE];  // Bs[.][k][c] = B[k0 + k][c0 + c]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int pt, ct;
-  if (!xcd_tile(g, ldb / (16 * NB), (int)(Npad / DPT), pt, ct)) return;
+  if (!xcd_tile(blockIdx.x, ldb / TILE, (int)(Npad / DPT), pt, ct)) return;
   const long p0 = (long)pt * DPT;
-  const int c0 = ct * 16 * NB;
-  // this thread's share of a stage: Phi row (tid / 2), 8 columns from (tid % 2) * 8;
-  // B elements tid + q * 256 (q < NB) of the 16 x 16 NB stage
-  constexpr int HALF = DKS / 2, NA = HALF / 2, NBQ = NB * DKS / 16;
-  const double *arow = phi + (p0 + (tid >> 1)) * ld + (tid & 1) * HALF;
-  auto load = [&](d2 (&ra)[NA], double (&rb)[NBQ], int k0) {
+  const int c0 = ct * TILE, am = tid >> 1, ak = (tid & 1) * 8;
+  const double *arow = phi + (p0 + am) * ld + ak;
+  d2 ra[4];
+  double rb[4];
+  auto load = [&](int k0) {
 #pragma unroll
-    for (int i = 0; i < NA; ++i) ra[i] = *(const d2 *)(arow + k0 + 2 * i);
+    for (int i = 0; i < 4; ++i) ra[i] = *(const d2 *)(arow + k0 + 2 * i);
 #pragma unroll
-    for (int q = 0; q < NBQ; ++q) {
-      const int e = tid + q * 256, k = e / (16 * NB), c = e % (16 * NB);
-      rb[q] = B[(long)(k0 + k) * ldb + c0 + c];
-    }
+    for (int q = 0; q < 4; ++q) rb[q] = B[(long)(k0 + (tid + q * 256) / TILE) * ldb + c0 + tid % TILE];
   };
-  auto store = [&](const d2 (&ra)[NA], const double (&rb)[NBQ], int buf) {
-    const int m = tid >> 1, kb = (tid & 1) * HALF;
+  auto store = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < NA; ++i) {
-      As[buf][kb + 2 * i][m] = ra[i].x;
-      As[buf][kb + 2 * i + 1][m] = ra[i].y;
-    }
+    for (int i = 0; i < 4; ++i) As[buf][ak + 2 * i][am] = ra[i].x, As[buf][ak + 2 * i + 1][am] = ra[i].y;
 #pragma unroll
-    for (int q = 0; q < NBQ; ++q) {
-      const int e = tid + q * 256, k = e / (16 * NB), c = e % (16 * NB);
-      Bs[buf][k][c] = rb[q];
-    }
+    for (int q = 0; q < 4; ++q) Bs[buf][(tid + q * 256) / TILE][tid % TILE] = rb[q];
   };
-  d4 acc[2][NB];
+  d4 acc[2][4];
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
-    for (int b = 0; b < NB; ++b) acc[a][b] = (d4){0, 0, 0, 0};
+    for (int b = 0; b < 4; ++b) acc[a][b] = (d4){0, 0, 0, 0};
   const int kr = lane >> 4, mi = lane & 15;
-  auto compute = [&](int buf) {
+  load(0);
+  store(0);
+  __syncthreads();
+  for (int k0 = 0; k0 < ld; k0 += DKS) {
+    const int buf = (k0 / DKS) & 1;
+    if (k0 + DKS < ld) load(k0 + DKS);
 #pragma unroll
     for (int ks = 0; ks < DKS; ks += 4) {
-      double a[2], b[NB];
+      double a[2], b[4];
 #pragma unroll
       for (int i = 0; i < 2; ++i) a[i] = As[buf][ks + kr][wave * 32 + i * 16 + mi];
 #pragma unroll
-      for (int j = 0; j < NB; ++j) b[j] = Bs[buf][ks + kr][j * 16 + mi];
+      for (int j = 0; j < 4; ++j) b[j] = Bs[buf][ks + kr][j * 16 + mi];
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < NB; ++j)
+        for (int j = 0; j < 4; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
     }
-  };
-  const int nstage = kend / DKS;  // K stages holding real functions (the rest are zero padding)
-  d2 ra0[NA], ra1[NA];
-  double rb0[NBQ], rb1[NBQ];
-  if (PF == 1) {
-    // one stage in flight: load st + 1 while computing st
-    load(ra0, rb0, 0);
-    store(ra0, rb0, 0);
+    if (k0 + DKS < ld) store(buf ^ 1);
     __syncthreads();
-    for (int st = 0; st < nstage; ++st) {
-      const int buf = st & 1;
-      if (st + 1 < nstage) load(ra0, rb0, (st + 1) * DKS);
-      compute(buf);
-      if (st + 1 < nstage) store(ra0, rb0, buf ^ 1);
-      __syncthreads();
-    }
-  } else {
-    // two stages in flight: registers hold st + 1 (to store) and st + 2 (arriving) while
-    // stage st is computed from LDS
-    load(ra0, rb0, 0);
-    store(ra0, rb0, 0);
-    if (nstage > 1) load(ra1, rb1, DKS);
-    __syncthreads();
-    for (int st = 0; st < nstage; st += 2) {
-      if (st + 2 < nstage) load(ra0, rb0, (st + 2) * DKS);
-      compute(0);
-      if (st + 1 < nstage) store(ra1, rb1, 1);
-      __syncthreads();
-      if (st + 1 >= nstage) break;
-      if (st + 3 < nstage) load(ra1, rb1, (st + 3) * DKS);
-      compute(1);
-      if (st + 2 < nstage) store(ra0, rb0, 0);
-      __syncthreads();
-    }
   }
   // f64 16x16x4 output: lane i, element r -> row (i / 16) + 4 r, column i % 16
-  if (MODE == MODE_STORE_X) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const long p = p0 + wave * 32 + i * 16 + kr + 4 * r;
-#pragma unroll
-        for (int j = 0; j < NB; ++j) partial[p * ldb + c0 + j * 16 + mi] = acc[i][j][r];
-      }
-    return;
-  }
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const long p = p0 + wave * 32 + i * 16 + kr + 4 * r;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) X[p * ldb + c0 + j * 16 + mi] = acc[i][j][r];
+    }
+}
+
+// -------------------------------------------------------------- density over column tiles
+// rho = diag(Phi P Phi^T) takes only the symmetric part of P, so P is folded onto the lower
+// block triangle (16 x 16 blocks): Q_kc = P_kc + P_ck for block row k below block column c, P
+// itself in the diagonal blocks, nothing above; rho_p = sum_c Phi_pc (Phi Q)_pc. Column tile ct
+// (64 columns) then multiplies the functions from 64 ct on only, and inside its diagonal the
+// blocks k >= c: nb (nb + 1) / 2 blocks instead of nb^2.
+//
+// The operand (Q, or C in the orbital form) is laid out in fragment order, per column tile and
+// group of 16 k: [ct][g][j][h][lane][2], lane (kr, mi) of block j holding k = 16 g + 4 kr + 2 h
+// + (0, 1), column 64 ct + 16 j + mi.
+__host__ __device__ inline long operand_size(int groups, int ntile) { return (long)ntile * groups * 1024; }
+
+__device__ __forceinline__ void density_operand_body(const double *__restrict__ src, int n, int ncol, int fold,
+                                                     int groups, double *__restrict__ dst, long e) {
+  const int t = (int)(e & 1), lane = (int)(e >> 1) & 63, h = (int)(e >> 7) & 1, j = (int)(e >> 8) & 3;
+  const long gg = e >> 10;
+  const int g = (int)(gg % groups), ct = (int)(gg / groups);
+  const int k = 16 * g + 4 * (lane >> 4) + 2 * h + t, c = 64 * ct + 16 * j + (lane & 15);
+  double v = 0.0;
+  if (k < n && c < ncol) {
+    if (!fold)
+      v = src[(long)k * ncol + c];
+    else if (g == 4 * ct + j)
+      v = src[(long)k * n + c];
+    else if (g > 4 * ct + j)
+      v = src[(long)k * n + c] + src[(long)c * n + k];
+  }
+  dst[e] = v;
+}
+
+__global__ void __launch_bounds__(256) k_density_operand(const double *__restrict__ src, int n, int ncol,
+                                                         int fold, int groups, long size,
+                                                         double *__restrict__ dst) {
+  const long e = (long)blockIdx.x * 256 + threadIdx.x;
+  if (e < size) density_operand_body(src, n, ncol, fold, groups, dst, e);
+}
+
+__global__ void __launch_bounds__(256) k_density_operand_group(const OperandMember *__restrict__ mem, int nmem) {
+  const long g = blockIdx.x;
+  const OperandMember &m = mem[group_member(mem, nmem, g)];
+  density_operand_body(m.P, m.n, m.n, 1, m.groups, m.dst, (g - m.block0) * 256 + threadIdx.x);
+}
+
+constexpr int DT_SG = 2;                     // k groups per LDS stage
+constexpr int DT_STAGE = DT_SG * 1024;       // doubles
+
+// Workgroup: 4 waves, wave w owns 16 RB rows of points and the tile's NB column blocks. Phi rows
+// come straight from memory as MFMA operands (lane (kr, mi) loads Phi[row mi][16 g + 4 kr .. + 3],
+// the next group's vectors in flight; the k order inside a group is permuted alike on both
+// operands), the operand through double-buffered LDS shared by the waves. Per group a wave issues
+// RB x NB x 4 products and RB + 2 NB loads, with constant offsets: FP64 MFMA holds the VALU, so
+// the loop has next to no other arithmetic. Bound by FP64 MFMA and by the start and end of each
+// workgroup. Measured: P form, n = 300, 472,000 points 1.95 -> 1.05 ms against 64-column tiles
+// over the whole P staged through LDS on both sides; orbital form, n = 480, 90 orbitals,
+// 1,062,000 points 2.62 -> 2.07 ms (96 columns instead of 128).
+template <int RB, int NB, bool PFORM>
+__device__ __forceinline__ void density_tile_body(const DensityMember &d, int pt, int ct, double *lds) {
+  const int tid = threadIdx.x, lane = tid & 63, kr = lane >> 4, mi = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ld = d.ld, G = d.groups, g0 = PFORM ? 4 * ct : 0;
+  const long row0 = ((long)pt * 4 + wave) * 16 * RB;
+  const char *abase = (const char *)(d.phi + row0 * ld);  // wave-uniform; lane offsets below
+  unsigned aoff[RB];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) aoff[rb] = (unsigned)(((16 * rb + mi) * ld + 4 * kr) * 8);
+  const double *src = d.B + (long)ct * G * 1024;
+  d2 r[DT_SG * 2];
+  auto load = [&](int g) {  // operand of groups g, g + 1 (the last group again past the end)
+#pragma unroll
+    for (int q = 0; q < DT_SG * 2; ++q) {
+      const int gq = min(g + q / 2, G - 1);
+      r[q] = ((const d2 *)(src + (long)gq * 1024))[(q & 1) * 256 + tid];
+    }
+  };
+  auto store = [&](int buf) {
+#pragma unroll
+    for (int q = 0; q < DT_SG * 2; ++q) ((d2 *)(lds + buf * DT_STAGE))[q * 256 + tid] = r[q];
+  };
+  d4 acc[RB][NB], a[2][RB];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[rb][j] = (d4){0, 0, 0, 0};
+  auto rows = [&](int s, int g) {
+    const char *b = abase + (long)min(g, G - 1) * 128;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) a[s][rb] = *(const d4 *)(b + aoff[rb]);
+  };
+  // group gg of the stage, its first NJ column blocks
+  auto group = [&](auto NJ, int buf, int gg) {
+    constexpr int nj = decltype(NJ)::value < NB ? decltype(NJ)::value : NB;
+    d2 b[nj][2];
+#pragma unroll
+    for (int j = 0; j < nj; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        b[j][h] = ((const d2 *)(lds + buf * DT_STAGE + gg * 1024))[(j * 2 + h) * 64 + lane];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int j = 0; j < nj; ++j)
+          acc[rb][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[gg][rb][s], b[j][s >> 1][s & 1], acc[rb][j], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto stage = [&](auto NJ0, auto NJ1, int g, int buf) {
+    load(g + 2);
+    rows(1, g + 1);
+    group(NJ0, buf, 0);
+    rows(0, g + 2);
+    if (g + 1 < G) group(NJ1, buf, 1);
+    store(buf ^ 1);
+    __syncthreads();
+  };
+  load(g0);
+  rows(0, g0);
+  store(0);
+  __syncthreads();
+  typedef std::integral_constant<int, 1> N1;
+  typedef std::integral_constant<int, 2> N2;
+  typedef std::integral_constant<int, 3> N3;
+  typedef std::integral_constant<int, 4> N4;
+  int g = g0, buf = 0;
+  if (PFORM) {
+    stage(N1(), N2(), g, 0);
+    g += 2;
+    if (g < G) {
+      stage(N3(), N4(), g, 1);
+      g += 2;
+    }
+  }
+#pragma unroll 1
+  for (; g < G; g += 2, buf ^= 1) stage(N4(), N4(), g, buf);
+  // f64 16x16x4 output: lane i, element r -> row (i / 16) + 4 r, column i % 16
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const long p = row0 + rb * 16 + kr + 4 * q;
       double sum = 0.0;
 #pragma unroll
       for (int j = 0; j < NB; ++j) {
-        const double x = acc[i][j][r];
-        sum += MODE == MODE_ORB ? x * x : x * phi[p * ld + c0 + j * 16 + mi];
+        const double x = acc[rb][j][q];
+        sum += PFORM ? x * d.phi[p * ld + 64 * ct + j * 16 + mi] : x * x;
       }
       sum += __shfl_xor(sum, 8);
       sum += __shfl_xor(sum, 4);
       sum += __shfl_xor(sum, 2);
       sum += __shfl_xor(sum, 1);
-      if (mi == 0 && p < nvalid) partial[(long)ct * Npad + p] = scale * sum;
+      if (mi == 0 && p < d.nvalid) d.partial[(long)ct * d.Npad + p] = d.scale * sum;
     }
 }
 
-template <int NB, int MODE, int DKS, int PF>
-__global__ void __launch_bounds__(256) k_density_mfma(const double *__restrict__ phi, int ld,
-                                                      long Npad, const double *__restrict__ B,
-                                                      int ldb, int kend, double scale,
-                                                      long nvalid,
-                                                      double *__restrict__ partial) {
-  density_mfma_body<NB, MODE, DKS, PF>(phi, ld, Npad, B, ldb, kend, scale, nvalid, partial,
-                                       blockIdx.x);
+template <int RB, bool PFORM>
+__device__ __forceinline__ void density_tiles(const DensityMember &d, int g, double *lds) {
+  int pt, ct;
+  if (!xcd_tile(g, d.ntile, (int)(d.Npad / (64 * RB)), pt, ct)) return;
+  if constexpr (PFORM) {
+    density_tile_body<RB, 4, true>(d, pt, ct, lds);
+  } else {
+    // the last tile's own column blocks
+    switch (min(4, (d.ncol - 64 * ct + 15) / 16)) {
+      case 1: density_tile_body<RB, 1, false>(d, pt, ct, lds); break;
+      case 2: density_tile_body<RB, 2, false>(d, pt, ct, lds); break;
+      case 3: density_tile_body<RB, 3, false>(d, pt, ct, lds); break;
+      default: density_tile_body<RB, 4, false>(d, pt, ct, lds);
+    }
+  }
+}
+
+template <int RB, bool PFORM>
+__global__ void __launch_bounds__(256, RB == 4 ? 2 : 3) k_density_tiles(DensityMember d) {
+  __shared__ double lds[2 * DT_STAGE];
+  density_tiles<RB, PFORM>(d, blockIdx.x, lds);
 }
 
 // Many plans in one launch: workgroup blockIdx.x belongs to the member whose block range
 // holds it (block0 multiples of 8, so the XCD-aware tile order of each member is kept).
-template <int NB, int MODE, int DKS, int PF>
-__global__ void __launch_bounds__(256) k_density_mfma_group(const DensityMember *__restrict__ mem,
-                                                            int nmem) {
+__global__ void __launch_bounds__(256, 3) k_density_tiles_group(const DensityMember *__restrict__ mem, int nmem) {
+  __shared__ double lds[2 * DT_STAGE];
   const long g = blockIdx.x;
-  const DensityMember &d = mem[group_member(mem, nmem, g)];
-  density_mfma_body<NB, MODE, DKS, PF>(d.phi, d.ld, d.Npad, d.B, d.ldb, d.kend, d.scale, d.nvalid,
-                                       d.partial, (int)(g - d.block0));
+  const DensityMember d = mem[group_member(mem, nmem, g)];
+  density_tiles<2, true>(d, (int)(g - d.block0), lds);
 }
 
 // Orbital form with C resident in LDS: the whole zero-padded C [kend x 16 NB] is copied
@@ -401,78 +503,66 @@ void launch_orb_stream_nb(const double *phi, int ld, long Npad, const double *C,
     launch_orb_stream_scr<NB, RB, WAVES, PF, false>(phi, ld, Npad, C, nrow, ncol, kend, scale, nvalid, out, sc, s);
 }
 
-template <int MODE, int DKS, int PF>
-void launch_density_ks(int nb, dim3 tiles, const double *phi, int ld, long Npad, const double *B,
-                       int ldb, int nreal, double scale, long nvalid, double *partial,
-                       hipStream_t s) {
-  // tiles = (point tiles, column tiles) -> one 1-D grid in the XCD-aware order
-  const dim3 grid((unsigned)(round_up(tiles.x, 8) * tiles.y));
-  // Phi columns and B rows from nreal on are zero: the K loop stops at the first stage
-  // boundary past them (the skipped products are exact zeros)
-  const int kend = (nreal > 0 && nreal < ld) ? (int)std::min<long>(ld, round_up(nreal, DKS)) : ld;
-  switch (nb) {
-    case 1: k_density_mfma<1, MODE, DKS, PF><<<grid, 256, 0, s>>>(phi, ld, Npad, B, ldb, kend, scale, nvalid, partial); break;
-    case 2: k_density_mfma<2, MODE, DKS, PF><<<grid, 256, 0, s>>>(phi, ld, Npad, B, ldb, kend, scale, nvalid, partial); break;
-    case 3: k_density_mfma<3, MODE, DKS, PF><<<grid, 256, 0, s>>>(phi, ld, Npad, B, ldb, kend, scale, nvalid, partial); break;
-    default: k_density_mfma<4, MODE, DKS, PF><<<grid, 256, 0, s>>>(phi, ld, Npad, B, ldb, kend, scale, nvalid, partial); break;
-  }
-  NAPMO_HIP(hipGetLastError());
-}
-
-// ks: K per stage, 16 or 32 (32 needs ld % 32 == 0); pf: stages in flight, 1 or 2
-template <int MODE>
-void launch_density_nb(int nb, dim3 grid, const double *phi, int ld, long Npad, const double *B,
-                       int ldb, double *partial, hipStream_t s, int ks = 16, int pf = 1,
-                       int nreal = 0, double scale = 1.0, long nvalid = -1) {
-  if (nvalid < 0) nvalid = Npad;
-  if (ks == 32 && ld % 32 == 0) {
-    if (pf == 2)
-      launch_density_ks<MODE, 32, 2>(nb, grid, phi, ld, Npad, B, ldb, nreal, scale, nvalid, partial, s);
-    else
-      launch_density_ks<MODE, 32, 1>(nb, grid, phi, ld, Npad, B, ldb, nreal, scale, nvalid, partial, s);
-  } else {
-    if (pf == 2)
-      launch_density_ks<MODE, 16, 2>(nb, grid, phi, ld, Npad, B, ldb, nreal, scale, nvalid, partial, s);
-    else
-      launch_density_ks<MODE, 16, 1>(nb, grid, phi, ld, Npad, B, ldb, nreal, scale, nvalid, partial, s);
-  }
-}
-
 }  // namespace
 
-long density_group_fill(DensityMember &d, const double *phi, int ld, long Npad, const double *P,
-                        double *partial, int nreal, int ks, long block0) {
-  NAPMO_REQUIRE(ld % TILE == 0 && Npad % DPT == 0 && block0 % 8 == 0, "grouped density: padding");
-  const int dks = (ks == 32 && ld % 32 == 0) ? 32 : 16;
-  d.phi = phi, d.B = P, d.partial = partial, d.Npad = Npad, d.nvalid = Npad, d.block0 = block0;
-  d.ld = ld, d.ldb = ld, d.scale = 1.0;
-  d.kend = (nreal > 0 && nreal < ld) ? (int)std::min<long>(ld, round_up(nreal, dks)) : ld;
-  return round_up(Npad / DPT, 8) * (ld / TILE);
+static DensityMember density_member(const double *phi, int ld, long Npad, const double *B, int n, int ncol,
+                                    int ntile, double *partial, double scale, long nvalid) {
+  NAPMO_REQUIRE(ld % TILE == 0 && Npad % 256 == 0 && n >= 1 && n <= ld, "density: padding mismatch");
+  DensityMember d = {};
+  d.phi = phi, d.B = B, d.partial = partial, d.Npad = Npad, d.nvalid = nvalid, d.scale = scale;
+  d.ld = ld, d.groups = (int)div_up(n, 16), d.ntile = ntile, d.ncol = ncol;
+  return d;
 }
 
-void launch_density_group(const DensityMember *d_mem, int nmem, long nblocks, int ks, int pf,
-                          hipStream_t s) {
-  if (nmem <= 0 || nblocks <= 0) return;
-  const dim3 grid((unsigned)nblocks);
-  if (ks == 32) {
-    if (pf == 2)
-      k_density_mfma_group<4, MODE_P, 32, 2><<<grid, 256, 0, s>>>(d_mem, nmem);
-    else
-      k_density_mfma_group<4, MODE_P, 32, 1><<<grid, 256, 0, s>>>(d_mem, nmem);
-  } else {
-    if (pf == 2)
-      k_density_mfma_group<4, MODE_P, 16, 2><<<grid, 256, 0, s>>>(d_mem, nmem);
-    else
-      k_density_mfma_group<4, MODE_P, 16, 1><<<grid, 256, 0, s>>>(d_mem, nmem);
-  }
+long density_operand_size(int n, int ncol) {
+  return operand_size((int)div_up(n, 16), (int)div_up(ncol, 64));
+}
+
+void launch_density_operand(const double *src, int n, int ncol, bool fold, double *dst, hipStream_t s) {
+  const long size = density_operand_size(n, ncol);
+  k_density_operand<<<div_up(size, 256), 256, 0, s>>>(src, n, ncol, fold ? 1 : 0, (int)div_up(n, 16), size, dst);
   NAPMO_HIP(hipGetLastError());
 }
 
-void launch_density_f64(const double *phi, int ld, long Npad, const double *P, double *partial,
-                        hipStream_t s, int ks, int pf, int nreal) {
-  NAPMO_REQUIRE(ld % TILE == 0 && Npad % DPT == 0, "density: padding mismatch");
-  launch_density_nb<MODE_P>(4, dim3(Npad / DPT, ld / TILE), phi, ld, Npad, P, ld, partial, s, ks,
-                            pf, nreal);
+long density_operand_group_fill(OperandMember &m, const double *P, int n, double *dst, long block0) {
+  m.P = P, m.dst = dst, m.block0 = block0, m.n = n, m.groups = (int)div_up(n, 16);
+  return density_operand_size(n, n) / 256;
+}
+
+void launch_density_operand_group(const OperandMember *d_mem, int nmem, long nblocks, hipStream_t st) {
+  if (nmem <= 0 || nblocks <= 0) return;
+  k_density_operand_group<<<dim3((unsigned)nblocks), 256, 0, st>>>(d_mem, nmem);
+  NAPMO_HIP(hipGetLastError());
+}
+
+// Points per workgroup: 256 (64 per wave, the fewest operand reads per product) where that makes
+// at least two rounds of the 512 workgroups the device holds, else 128.
+template <bool PFORM>
+static void launch_density_tiles(const DensityMember &d, hipStream_t s) {
+  if (d.Npad / 256 * d.ntile >= 1024)
+    k_density_tiles<4, PFORM><<<(unsigned)(round_up(d.Npad / 256, 8) * d.ntile), 256, 0, s>>>(d);
+  else
+    k_density_tiles<2, PFORM><<<(unsigned)(round_up(d.Npad / 128, 8) * d.ntile), 256, 0, s>>>(d);
+  NAPMO_HIP(hipGetLastError());
+}
+
+long density_group_fill(DensityMember &d, const double *phi, int ld, long Npad, const double *operand,
+                        double *partial, int n, long block0) {
+  NAPMO_REQUIRE(block0 % 8 == 0, "grouped density: workgroup alignment");
+  d = density_member(phi, ld, Npad, operand, n, n, (int)div_up(n, 64), partial, 1.0, Npad);
+  d.block0 = block0;
+  return round_up(Npad / 128, 8) * d.ntile;
+}
+
+void launch_density_group(const DensityMember *d_mem, int nmem, long nblocks, hipStream_t s) {
+  if (nmem <= 0 || nblocks <= 0) return;
+  k_density_tiles_group<<<dim3((unsigned)nblocks), 256, 0, s>>>(d_mem, nmem);
+  NAPMO_HIP(hipGetLastError());
+}
+
+void launch_density_f64(const double *phi, int ld, long Npad, const double *operand, double *partial,
+                        hipStream_t s, int n) {
+  launch_density_tiles<true>(density_member(phi, ld, Npad, operand, n, n, (int)div_up(n, 64), partial, 1.0, Npad), s);
 }
 
 int density_orb_cols(int nocc) {
@@ -480,18 +570,12 @@ int density_orb_cols(int nocc) {
   return c <= 64 ? c : (int)round_up(nocc, 64);
 }
 
-int density_orb_tiles(int ldc) { return ldc <= 64 ? 1 : ldc / 64; }
-
-void launch_density_orb_f64(const double *phi, int ld, long Npad, const double *C, int ldc,
-                            double *partial, hipStream_t s, int ks, int pf, int nreal, double scale,
-                            long nvalid) {
-  NAPMO_REQUIRE(Npad % DPT == 0 && ld % 16 == 0 && ldc % 16 == 0, "density_orb: padding");
-  const int nb = ldc <= 64 ? ldc / 16 : 4;
-  NAPMO_REQUIRE(ldc <= 64 || ldc % 64 == 0, "density_orb: orbital padding");
-  NAPMO_REQUIRE(nvalid < 0 || density_orb_tiles(ldc) == 1,
-                "density_orb: a direct (scaled) write needs one column tile");
-  launch_density_nb<MODE_ORB>(nb, dim3(Npad / DPT, density_orb_tiles(ldc)), phi, ld, Npad, C, ldc,
-                              partial, s, ks, pf, nreal, scale, nvalid);
+void launch_density_orb_f64(const double *phi, int ld, long Npad, const double *operand, int n, int nocc,
+                            double *partial, hipStream_t s, double scale, long nvalid) {
+  const int ntile = (int)div_up(nocc, 64);
+  NAPMO_REQUIRE(nvalid < 0 || ntile == 1, "density_orb: a direct (scaled) write needs one column tile");
+  launch_density_tiles<false>(density_member(phi, ld, Npad, operand, n, nocc, ntile, partial, scale,
+                                             nvalid < 0 ? Npad : nvalid), s);
 }
 
 bool density_orb_stream_supported(int ld, int ldc, int nreal) {
@@ -568,7 +652,8 @@ void launch_permute_cols(const double *phi, int ld, long Npad, const int *perm, 
 void launch_phi_times(const double *phi, int ld, long Npad, const double *B, int ldb, double *X,
                       hipStream_t s) {
   NAPMO_REQUIRE(ld % TILE == 0 && ldb % TILE == 0 && Npad % DPT == 0, "phi_times: padding");
-  launch_density_nb<MODE_STORE_X>(4, dim3(Npad / DPT, ldb / TILE), phi, ld, Npad, B, ldb, X, s);
+  k_phi_times<<<(unsigned)(round_up(Npad / DPT, 8) * (ldb / TILE)), 256, 0, s>>>(phi, ld, Npad, B, ldb, X);
+  NAPMO_HIP(hipGetLastError());
 }
 
 }  // namespace napmo

@@ -222,10 +222,9 @@ int FockPlan::profile_read(double *avg_ms, int nphase) {
 
 void FockPlan::density_P(int slot, const double *dP) {
   hipStream_t st = stream;
-  // P (n x n) into the zero-padded ld x ld operand (a kernel, so the build can be captured)
-  launch_pad2d(dP, n, n, P.get(), ld, ld, st);
+  launch_density_operand(dP, n, n, true, P.get(), st);
   mark(slot, 0);
-  launch_density_f64(phi64.get(), ld, Npad, P.get(), rho_part.get(), st, density_ks, density_pf, n);
+  launch_density_f64(phi64.get(), ld, Npad, P.get(), rho_part.get(), st, n);
   mark(slot, 1);
   launch_rho_reduce(rho_part.get(), ld / TILE, Npad, grid.N, rho.get(), st);
 }
@@ -272,7 +271,7 @@ void FockPlan::density_screen_setup() {
 void FockPlan::density_C(int slot, const double *dC, int nocc, double eta) {
   NAPMO_REQUIRE(nocc > 0 && nocc <= n, "orbital count out of range");
   hipStream_t st = stream;
-  const int ldc = density_orb_cols(nocc), nct = density_orb_tiles(ldc);
+  const int ldc = density_orb_cols(nocc), nct = (int)div_up(nocc, 64);
   Pfull.resize((size_t)n * n);
   if (nct == 1 && density_stream && density_orb_stream_supported(ld, ldc, n)) {
     // C resident in LDS (read as given, no padded copy), Phi streamed; the epilogue writes
@@ -286,19 +285,17 @@ void FockPlan::density_C(int slot, const double *dC, int nocc, double eta) {
     mark(slot, 1);
     return;
   }
-  Cpad.resize((size_t)ld * ldc);
+  Cpad.resize(density_operand_size(n, nocc));
   if (rho_part.size() < (size_t)nct * Npad) rho_part.resize((size_t)nct * Npad);
-  launch_pad2d(dC, n, nocc, Cpad.get(), ld, ldc, st);
+  launch_density_operand(dC, n, nocc, false, Cpad.get(), st);
   launch_gram(dC, n, nocc, eta, Pfull.get(), st);
   mark(slot, 0);
   if (nct == 1) {
     // one column tile: the kernel's epilogue writes rho = eta sum_i X_pi^2 itself
-    launch_density_orb_f64(phi64.get(), ld, Npad, Cpad.get(), ldc, rho.get(), st, density_ks,
-                           density_pf, n, eta, grid.N);
+    launch_density_orb_f64(phi64.get(), ld, Npad, Cpad.get(), n, nocc, rho.get(), st, eta, grid.N);
     mark(slot, 1);
   } else {
-    launch_density_orb_f64(phi64.get(), ld, Npad, Cpad.get(), ldc, rho_part.get(), st, density_ks,
-                           density_pf, n);
+    launch_density_orb_f64(phi64.get(), ld, Npad, Cpad.get(), n, nocc, rho_part.get(), st);
     mark(slot, 1);
     launch_rho_reduce(rho_part.get(), nct, Npad, grid.N, rho.get(), st, eta);
   }

@@ -54,8 +54,8 @@ struct FockPlan {
   std::pair<long, long> int8_screen_stats();
   int use_pass = 0;  // 0: per-tile kernels, 1: one-pass BF16x3, 2: symmetric one-pass BF16x3
   long fock_wg = 0, pass_wg = 0;  // workgroup targets of the two shapes (0 = default)
-  int density_ks = 16;            // K per LDS stage of the density kernels (16 or 32)
-  int density_pf = 1;             // stages in flight in the density kernels (1 or 2)
+  int density_ks = 16;            // NAPMO_TUNE_DENSITY_KS: kept, unused
+  int density_pf = 1;             // NAPMO_TUNE_DENSITY_PF: kept, unused
   int density_stream = 1;  // orbital form: C resident in LDS, Phi streamed (when it fits), in
                            // launch shape 1..3; 0: the LDS-staged kernels
   int density_screen = 0;  // NAPMO_TUNE_DENSITY_SCREEN (0: off)

@@ -139,12 +139,6 @@ GroupPlan::GroupPlan(const std::vector<FockPlan *> &ps, const std::vector<double
   PoissonPlan &pl = ug.plan(lmax);
   NAPMO_REQUIRE(pl.work.T.size() >= (size_t)tsize, "group plan: synthesis table size");
   // member tables that do not depend on the build's pointers
-  // the density stage shape most of the plans were tuned to (it does not change results)
-  std::map<std::pair<int, int>, int> votes;
-  for (auto *q : plans) ++votes[{q->density_ks, q->density_pf}];
-  int best = -1;
-  for (const auto &kv : votes)
-    if (kv.second > best) best = kv.second, ks = kv.first.first, pf = kv.first.second;
   std::vector<DensityMember> dm(nm);
   std::vector<RhoReduceMember> rm(nm);
   std::vector<ScaleMember> sm(nm);
@@ -153,7 +147,7 @@ GroupPlan::GroupPlan(const std::vector<FockPlan *> &ps, const std::vector<double
     FockPlan &q = *plans[m];
     const long N = q.grid.N;
     dens_blocks += density_group_fill(dm[m], q.phi64.get(), q.ld, q.Npad, q.P.get(), q.rho_part.get(),
-                                      q.n, ks, dens_blocks);
+                                      q.n, dens_blocks);
     rm[m] = RhoReduceMember{q.rho_part.get(), rho.get() + p0[m], q.Npad, N, rho_blocks, q.ld / TILE};
     rho_blocks += div_up(N, 256);
     sm[m] = ScaleMember{q.s.get(), p0[m], N, q.Npad, scale_blocks, A0[m], A0[m + 1]};
@@ -195,7 +189,7 @@ void GroupPlan::io_tables(IoTables &io, const double *const *dP, double *const *
   for (int m = 0; same && m < nm; ++m)
     same = io.P[m] == dP[m] && io.F[m] == dF[m] && io.E[m] == dE[m];
   if (same) return;
-  std::vector<PadMember> pm(nm);
+  std::vector<OperandMember> pm(nm);
   std::vector<FockReduceMember> frm(nm);
   std::vector<TraceMember> tm(nm), t2m(nm);
   std::vector<ApmoEnergyMember> em(nm);
@@ -203,8 +197,7 @@ void GroupPlan::io_tables(IoTables &io, const double *const *dP, double *const *
   for (int m = 0; m < nm; ++m) {
     FockPlan &q = *plans[m];
     NAPMO_REQUIRE(dP[m] && dF[m] && dE[m], "group build: null pointer");
-    pm[m] = PadMember{dP[m], q.P.get(), pad_blocks, q.n, q.n, q.ld, q.ld};
-    pad_blocks += div_up((long)q.ld * q.ld, 256);
+    pad_blocks += density_operand_group_fill(pm[m], dP[m], q.n, q.P.get(), pad_blocks);
     fred_blocks += fock_reduce_group_fill(frm[m], q.dsh, q.F_part.get(), q.n, dF[m], fred_blocks);
     const double *vs = coupled ? veff.get() : v.get();
     tm[m] = TraceMember{dP[m], dF[m], ug.wbw.get() + p0[m], rho.get() + p0[m], vs + p0[m],
@@ -235,8 +228,8 @@ void GroupPlan::io_tables(IoTables &io, const double *const *dP, double *const *
 
 void GroupPlan::launches(const IoTables &io) {
   const int nm = (int)plans.size();
-  launch_pad_group(io.pmem.get(), nm, io.pad_blocks, stream);
-  launch_density_group(dmem.get(), nm, dens_blocks, ks, pf, stream);
+  launch_density_operand_group(io.pmem.get(), nm, io.pad_blocks, stream);
+  launch_density_group(dmem.get(), nm, dens_blocks, stream);
   launch_rho_reduce_group(rmem.get(), nm, rho_blocks, stream);
   PoissonPlan &pl = ug.plan(lmax);
   AtomTables at = ug.tables(pl);

@@ -31,7 +31,6 @@ struct GroupPlan {
   };
   std::vector<SynthRange> ranges;
   DeviceBuffer<double> rho, v;    // [ug.N]
-  int ks = 16, pf = 1;            // density stage shape (does not change results)
   // member tables (device) and workgroup counts of the grouped launches
   DeviceBuffer<DensityMember> dmem;
   DeviceBuffer<RhoReduceMember> rmem;
@@ -49,7 +48,7 @@ struct GroupPlan {
   // the captured graph (which reads its tables at every replay, so eager builds on other
   // pointers must not rewrite them)
   struct IoTables {
-    DeviceBuffer<PadMember> pmem;
+    DeviceBuffer<OperandMember> pmem;
     DeviceBuffer<FockReduceMember> frmem;
     DeviceBuffer<TraceMember> tmem, t2mem;
     DeviceBuffer<ApmoEnergyMember> emem;

@@ -227,11 +227,15 @@ void launch_epc17_2_pairs_noalloc(const double *rE, const double *rN, const int 
                                   long Na, long Nb, const double *wbwN, double *vE, double *vN,
                                   double *energy, hipStream_t st);
 
-// rho[p] = Phi_p^T P Phi_p with FP64 MFMA (P [ld x ld] zero padded). partial [ntile x Npad].
-// nreal: functions actually present (columns nreal .. ld - 1 of Phi and rows of P are zero),
-// 0 = ld.
-void launch_density_f64(const double *phi, int ld, long Npad, const double *P, double *partial,
-                        hipStream_t s, int ks = 16, int pf = 1, int nreal = 0);
+// rho partials [ceil(n / 64) x Npad] of rho[p] = Phi_p^T P Phi_p with FP64 MFMA; operand from
+// launch_density_operand(P, n, n, fold = true).
+void launch_density_f64(const double *phi, int ld, long Npad, const double *operand, double *partial,
+                        hipStream_t s, int n);
+// The MFMA operand of P [n x n] folded onto its lower block triangle (fold) or of C [n x ncol], in
+// fragment order (density.hip): density_operand_size(n, ncol) doubles, at most
+// round_up(n, 64) round_up(ncol, 64).
+long density_operand_size(int n, int ncol);
+void launch_density_operand(const double *src, int n, int ncol, bool fold, double *dst, hipStream_t s);
 // rho[p] = scale * sum_t partial[t][p] for p < N.
 void launch_rho_reduce(const double *partial, int ntile, long Npad, long N, double *rho,
                        hipStream_t s, double scale = 1.0);
@@ -296,8 +300,7 @@ void launch_fock_syrk_pass(const FockShape &sh, const float *phi32, const double
 void launch_fock_bf16x3_pass(const FockShape &sh, const unsigned short *Ahi,
                              const unsigned short *Alo, const double *s, float *partial,
                              hipStream_t st);
-// partial[ct][p] = sum over orbital tile ct of (Phi C)_pi^2, C zero-padded [ld x ldc];
-// ldc = density_orb_cols(nocc), density_orb_tiles(ldc) partial rows.
+// columns of C padded to whole MFMA blocks
 int density_orb_cols(int nocc);
 // X [Npad x ldb] = Phi [Npad x ld] B [ld x ldb] on FP64 MFMA (ld, ldb multiples of 64).
 void launch_phi_times(const double *phi, int ld, long Npad, const double *B, int ldb, double *X,
@@ -321,12 +324,11 @@ void launch_grad_basis_part(const double *x, const double *y, const double *z, l
                             double *partial, hipStream_t st);
 void launch_grad_reduce(const double *partial, int n, long Ntotal, const int *centre_of,
                         int ncentre, double *grad, hipStream_t st);
-int density_orb_tiles(int ldc);
-// With one column tile (ldc <= 64), nvalid >= 0 makes the kernel write
-// partial[p] = scale * sum for p < nvalid directly (rho itself, no reduction pass).
-void launch_density_orb_f64(const double *phi, int ld, long Npad, const double *C, int ldc,
-                            double *partial, hipStream_t s, int ks = 16, int pf = 1, int nreal = 0,
-                            double scale = 1.0, long nvalid = -1);
+// partial[ct][p] = sum over the 64-orbital tile ct of (Phi C)_pi^2, operand from
+// launch_density_operand(C, n, nocc, fold = false). With one tile (nocc <= 64), nvalid >= 0 makes
+// the kernel write partial[p] = scale * sum for p < nvalid directly (rho itself).
+void launch_density_orb_f64(const double *phi, int ld, long Npad, const double *operand, int n, int nocc,
+                            double *partial, hipStream_t s, double scale = 1.0, long nvalid = -1);
 // Orbital form with all of C [nrow x ncol] (row-major as given, ncol <= 64, zero-padded to
 // 16-column blocks in LDS) resident in LDS, Phi streamed into MFMA operands:
 // out[p] = scale sum_c X_pc^2 for p < nvalid (nvalid < 0: Npad). shape 1..3: (rows per
@@ -358,12 +360,18 @@ void launch_selftest_mfma(int which, double *out, hipStream_t s);
 // ---- grouped launches: many plans (independent molecules) in one launch per phase. Each
 // member carries its own arguments; block0 is its first workgroup (a multiple of 8 where
 // the kernel orders tiles by XCD), and a workgroup finds its member by binary search.
-struct DensityMember {   // P-form density of one plan
+struct DensityMember {   // density over column tiles of one plan (B: the MFMA operand)
   const double *phi, *B;
   double *partial;
   long Npad, nvalid, block0;
-  int ld, ldb, kend;
+  int ld, groups, ntile, ncol;
   double scale;
+};
+struct OperandMember {   // the folded operand of one plan's P
+  const double *P;
+  double *dst;
+  long block0;
+  int n, groups;
 };
 struct FockMember {      // FP64 Fock partials of one plan
   const double *X, *s;
@@ -381,12 +389,6 @@ struct TraceMember {     // E[0] = 1/2 sum P o F, E[1] = 1/2 sum wbw rho v
   const double *P, *F, *wbw, *rho, *v;
   double *E, *work;
   long nn, N;
-};
-struct PadMember {       // src [rows x cols] -> dst [drows x dcols], zero padded
-  const double *src;
-  double *dst;
-  long block0;
-  int rows, cols, drows, dcols;
 };
 struct RhoReduceMember {  // rho[p] = sum_t partial[t][p], p < N
   const double *partial;
@@ -411,12 +413,12 @@ __host__ __device__ inline int group_member(const T *mem, int nmem, long g) {
   }
   return lo;
 }
-// Fills d for one plan's P-form density (ks as for launch_density_f64); returns its
-// workgroup count.
-long density_group_fill(DensityMember &d, const double *phi, int ld, long Npad, const double *P,
-                        double *partial, int nreal, int ks, long block0);
-void launch_density_group(const DensityMember *d_mem, int nmem, long nblocks, int ks, int pf,
-                          hipStream_t s);
+// Fill one plan's member; return its workgroup count.
+long density_operand_group_fill(OperandMember &m, const double *P, int n, double *dst, long block0);
+void launch_density_operand_group(const OperandMember *d_mem, int nmem, long nblocks, hipStream_t st);
+long density_group_fill(DensityMember &d, const double *phi, int ld, long Npad, const double *operand,
+                        double *partial, int n, long block0);
+void launch_density_group(const DensityMember *d_mem, int nmem, long nblocks, hipStream_t s);
 long fock_group_fill(FockMember &f, const FockShape &sh, const double *X, const double *s,
                      double *partial, long block0);
 // waves (4 or 8) and LDS of one member's workgroups: a launch takes members of one wave count,
@@ -428,7 +430,6 @@ long fock_reduce_group_fill(FockReduceMember &f, const FockShape &sh, const doub
                             double *F, long block0);
 void launch_fock_reduce_group(const FockReduceMember *d_mem, int nmem, long nblocks, hipStream_t st);
 void launch_traces_group(const TraceMember *d_mem, int nmem, hipStream_t st);
-void launch_pad_group(const PadMember *d_mem, int nmem, long nblocks, hipStream_t st);
 void launch_rho_reduce_group(const RhoReduceMember *d_mem, int nmem, long nblocks, hipStream_t st);
 // Coupled species (APMO), member m = species m with charge q_m: per union point p of m,
 // S_t = sum over t's centres of contrib[A Nu + p] (every species t, centres in order),
