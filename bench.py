@@ -231,12 +231,20 @@ SYNTH_MFMA_MIN_KEY = 9          # NAPMO_TUNE_SYNTH_MFMA_MIN
 
 def mfma_densities(grid, nset):
     """How many of nset densities the grid's many-density synthesis puts on MFMA: whole
-    tiles of 16 and a last tile of at least the grid's threshold."""
+    tiles of 16 and the rest in fours (at the default threshold 10, by what the rest costs
+    either way, as the library decides)."""
     thr = grid.get_tuning(SYNTH_MFMA_MIN_KEY)
+    rest = nset % 16
+    full = nset - rest
     if thr > 16:
         return 0
-    full, rest = 16 * (nset // 16), nset % 16
-    return full + (rest if rest >= thr else 0)
+    if thr != 10:
+        return nset if rest >= thr else full
+    if full == 0:
+        return nset if rest >= 12 else 0
+    if rest < 4:
+        return full
+    return nset - rest % 4 if rest % 4 <= 2 else nset
 
 
 def synth_roofline(phases, M, N, L, nset, n_mfma, traffic):

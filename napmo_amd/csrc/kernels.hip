@@ -910,34 +910,6 @@ void launch_contrib_reduce_tile(const double *tile, int M, long N, int nvalid, d
   NAPMO_HIP(hipGetLastError());
 }
 
-template <int LM>
-static void synth_mfma_dispatch(int lmax, hipStream_t s, const AtomTables &at, const double *geo,
-                                long N, const int *list, const int *wb, long nw, int ntile,
-                                const double *T, const double *aL, const double *aR,
-                                double *contrib) {
-  if constexpr (LM > MAX_LMAX) {
-    throw Error("lmax above the supported maximum " + std::to_string(MAX_LMAX));
-  } else {
-    if (lmax == LM)
-      launch_synth_mfma_t<LM>(s, at, geo, N, list, wb, nw, ntile, 16 * ntile, T, aL, aR,
-                              (long)at.M * N * 16, contrib);
-    else
-      synth_mfma_dispatch<LM + 1>(lmax, s, at, geo, N, list, wb, nw, ntile, T, aL, aR, contrib);
-  }
-}
-
-void launch_synth_mfma(const AtomTables &at, const double *geo, long N, const int *list,
-                       const int *wave_bucket, long nwaves, int ntile, const double *T,
-                       const double *ampL, const double *ampR, int lmax, double *contrib,
-                       hipStream_t s) {
-  NAPMO_REQUIRE(lmax >= 0 && lmax <= MAX_LMAX, "lmax out of range for synthesis");
-  NAPMO_REQUIRE(ntile >= 1 && ntile <= 4096, "MFMA synthesis: 1 to 4096 tiles of 16 densities");
-  if (nwaves <= 0) return;
-  synth_mfma_dispatch<0>(lmax, s, at, geo, N, list, wave_bucket, nwaves, ntile, T, ampL, ampR,
-                         contrib);
-  NAPMO_HIP(hipGetLastError());
-}
-
 __global__ void k_contrib_reduce_scale_group(const ScaleMember *__restrict__ mem, int nmem,
                                              const double *__restrict__ contrib,
                                              const long *__restrict__ cbase,

@@ -76,10 +76,11 @@ constexpr int SET_BATCH = 64;
 // MFMA synthesis: at most this many bytes of per-centre tile sums [M][N][16] at once (at
 // least one tile)
 constexpr long SYNTH_MFMA_BUDGET = 4L << 30;
-// A tile of 16 densities on MFMA costs about as much as ten one-density syntheses (2.7 ms
-// against 0.28 ms each on 16 centres x 472,000 points at lmax 12), so a last tile takes the
-// MFMA path from ten densities on.
+// NAPMO_TUNE_SYNTH_MFMA_MIN of a grid; the default stands for the rule of synth_mfma_count.
 constexpr int SYNTH_MFMA_MIN = 10;
+// How many of nset densities go through the MFMA synthesis: whole tiles of 16, the rest in fours
+// (13 to 15 as a padded tile).
+int synth_mfma_count(int nset, int min_tile);
 
 // Per-geometry pair buckets of the bucketed synthesis (see launch_synth2).
 struct SynthPairs {
@@ -186,9 +187,9 @@ struct DeviceGrid {
   DeviceBuffer<double> xchi, xdens, xaux;  // its workspace, kept between calls
   DeviceBuffer<double> xrho, xUy, xUdt;    // per batch of orbital pairs
   // Synthesis of nset densities on this grid from their radial solutions (set s at
-  // Uy, Udt + s ustride, plan(lmax) order): out[s ostride + p] = scale v_s[p]. Whole tiles
-  // of 16 densities, and a last tile of at least synth_mfma_min, go through the FP64 MFMA
-  // synthesis (launch_synth_mfma); the others one at a time through the bucketed synthesis.
+  // Uy, Udt + s ustride, plan(lmax) order): out[s ostride + p] = scale v_s[p]. The first
+  // synth_mfma_count go through the FP64 MFMA synthesis (launch_synth_mfma), the others one at a
+  // time through the bucketed synthesis.
   // Profiling phases 4 (tables), 5 (one-density synthesis), 7 (MFMA synthesis), 6 (centre
   // sums).
   void synth_sets(int lmax, int nset, const double *Uy, const double *Udt, long ustride,

@@ -1,5 +1,5 @@
-// The synthesis launchers (defined in synth_kernel.hpp and synth_mfma.hpp, instantiated per
-// lmax in synth_inst_*.hip) and the inverse radial transform they share with the pair lists.
+// The synthesis launchers (defined in synth_kernel.hpp, instantiated per lmax in
+// synth_inst_*.hip) and the inverse radial transform they share with the pair lists.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -23,10 +23,5 @@ template <int LMAX>
 void launch_synth2_t(int np, hipStream_t s, const AtomTables &at, const double *geo, long N,
                      const int *list, const int *wave_bucket, long nwaves, const double *T,
                      const double *aL, const double *aR, double *contrib);
-template <int LMAX>
-void launch_synth_mfma_t(hipStream_t s, const AtomTables &at, const double *geo, long N,
-                         const int *list, const int *wave_bucket, long nslots, int ntile,
-                         int ndp, const double *T, const double *aL, const double *aR,
-                         long tstride, double *contrib);
 
 }  // namespace napmo

@@ -116,3 +116,21 @@ def test_tile_boundaries(norb):
     d0 = run()
     assert np.array_equal(d0, run())
     print('norb %d: max|MFMA - one at a time| %.2e' % (norb, np.abs(a - b).max()))
+
+
+@pytest.mark.parametrize('lmax', [0, 1, 2, 7])
+@pytest.mark.parametrize('norb', [3, 12, 13, 19, 22, 36, 40, 47])
+def test_tiles_and_fours(norb, lmax):
+    # 0 to 2 tiles of 16 per launch with 0 to 3 fours (padded tile at 13; 47 = two launches),
+    # harmonic steps that are not a multiple of the loads in flight: the default split and
+    # everything on MFMA against one at a time, to the rounding of the bound above
+    import napmo_amd
+    g, _ = systems.gpu_system(ATOMS, [[]] * 3, 12, 26)
+    o, _ = systems.oracle_system(ATOMS, [[]] * 3, 12, 26)
+    phi, ri, V = _orbital_inputs(o, norb, 5)
+    doi, oi = np.linspace(0.02, -0.01, norb), np.linspace(-0.6, -0.3, norb)
+    run = lambda: napmo_amd.compute_dpsi(g, lmax, phi, doi, oi, ri, V, 1.0)  # noqa: E731
+    a, b = _both(g, run)
+    scale = np.abs(b).max(axis=1)
+    assert np.all(np.abs(a - b).max(axis=1) < 1e-13 * scale)
+    assert np.all(np.abs(run() - b).max(axis=1) < 1e-13 * scale)
