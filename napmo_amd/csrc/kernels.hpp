@@ -177,13 +177,14 @@ void launch_axpby(double a, const double *x, double b, const double *y, long N, 
 // Finite-element tables of one radial grid (helmholtz_tables in poisson_plan.cpp), per atom
 // offsets into concatenated arrays: c0 [2n x 7] band of the Galerkin matrix without the
 // a term, oa [2n x 7 x 6] a-term integrals, o2 [2n x 6] right-hand-side integrals of the
-// merged source f, j1 / j2 [sum nrad] (indexed like AtomTables::r).
+// merged source f, j1 / j2 [sum nrad] (indexed like AtomTables::r), sinv / supm [sum nrad]
+// 1 / pivots and eliminated super-diagonal of the spline-slope system.
 struct HelmholtzTables {
-  const double *c0, *oa, *o2, *j1, *j2;
+  const double *c0, *oa, *o2, *j1, *j2, *sinv, *supm;
   const long *c0_off, *oa_off, *o2_off;
 };
-// LDS of one radial system of n points: 2n x 13 band and multiplier doubles, 2n spline
-// factors and n/2 pivot words, and at least 3 columns of 2n: 280 n bytes (143 KB at 512)
+// LDS of one radial system of n points: 2n + 5 rows of 8 band entries and at least one
+// column, 4n + 2 doubles of coefficients and spline factors: 176 n + 376 bytes (90 KB at 512)
 constexpr int HELMHOLTZ_MAX_NRAD = 512;
 // out[o][p] = a[o][p] * s[o] - b[o][p] for norb rows of N points (s: device [norb]).
 void launch_scaled_diff(const double *a, const double *s, const double *b, int norb, long N,

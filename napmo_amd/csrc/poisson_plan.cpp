@@ -630,6 +630,7 @@ int DeviceGrid::profile_read(double *avg_ms, int nphase) {
 HelmholtzTables HelmholtzPlan::tables() const {
   HelmholtzTables t;
   t.c0 = c0.get(), t.oa = oa.get(), t.o2 = o2.get(), t.j1 = j1.get(), t.j2 = j2.get();
+  t.sinv = sinv.get(), t.supm = supm.get();
   t.c0_off = c0_off.get(), t.oa_off = oa_off.get(), t.o2_off = o2_off.get();
   return t;
 }
@@ -638,7 +639,7 @@ HelmholtzPlan &DeviceGrid::helmholtz() {
   if (hplan) return *hplan;
   require_atoms("orbital correction");
   auto h = std::make_unique<HelmholtzPlan>();
-  std::vector<double> c0, oa, o2, j1all, j2all;
+  std::vector<double> c0, oa, o2, j1all, j2all, sinv, supm;
   std::vector<long> c0o(M), oao(M), o2o(M);
   std::vector<std::pair<std::vector<double>, int>> seen;  // (radial grid key, first atom)
   for (int a = 0; a < M; ++a) {
@@ -650,6 +651,13 @@ HelmholtzPlan &DeviceGrid::helmholtz() {
     helmholtz_tables(at.rtf, tc0, toa, to2, tj1, tj2);
     j1all.insert(j1all.end(), tj1.begin(), tj1.end());
     j2all.insert(j2all.end(), tj2.begin(), tj2.end());
+    // elimination of the spline-slope system (2, 4, ..., 4, 2 | 1), unit off-diagonals
+    double upm = 0.0;
+    for (int i = 0; i < at.nrad; ++i) {
+      const double den = (i == 0 || i == at.nrad - 1 ? 2.0 : 4.0) - upm;
+      upm = i < at.nrad - 1 ? 1.0 / den : 0.0;
+      sinv.push_back(1.0 / den), supm.push_back(upm);
+    }
     std::vector<double> key = {(double)at.rtf.kind, at.rtf.p0, at.rtf.p1, (double)at.nrad};
     int first = -1;
     for (auto &s : seen)
@@ -666,6 +674,7 @@ HelmholtzPlan &DeviceGrid::helmholtz() {
   }
   h->c0.upload(c0, stream), h->oa.upload(oa, stream), h->o2.upload(o2, stream);
   h->j1.upload(j1all, stream), h->j2.upload(j2all, stream);
+  h->sinv.upload(sinv, stream), h->supm.upload(supm, stream);
   h->c0_off.upload(c0o, stream), h->oa_off.upload(oao, stream), h->o2_off.upload(o2o, stream);
   NAPMO_HIP(hipStreamSynchronize(stream));
   hplan = std::move(h);

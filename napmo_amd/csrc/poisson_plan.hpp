@@ -93,7 +93,7 @@ struct SynthPairs {
 
 // Orbital-correction tables of every atom (one copy per distinct radial grid).
 struct HelmholtzPlan {
-  DeviceBuffer<double> c0, oa, o2, j1, j2;
+  DeviceBuffer<double> c0, oa, o2, j1, j2, sinv, supm;
   DeviceBuffer<long> c0_off, oa_off, o2_off;
   HelmholtzTables tables() const;
 };
