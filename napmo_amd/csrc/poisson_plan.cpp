@@ -736,11 +736,9 @@ void DeviceGrid::exchange_potential(int ndim, const double *d_psi, const double 
   AtomTables at = tables(pl);
   // orbital pairs (s, v), v <= s, in order, SET_BATCH at a time: pair densities, their
   // projections and radial solves in one launch each, the synthesis of the batch
-  // (synth_sets), then per pair the accumulation into K
-  std::vector<std::pair<int, int>> prs;
-  for (int s = 0; s < ndim; ++s)
-    for (int v = 0; v <= s; ++v) prs.push_back({s, v});
-  const int npair = (int)prs.size(), nb = std::min(SET_BATCH, npair);
+  // (synth_sets), then its accumulation into K
+  const long npair = (long)ndim * (ndim + 1) / 2;
+  const int nb = (int)std::min<long>(SET_BATCH, npair);
   const int L = (lmax + 1) * (lmax + 1);
   long S = 0;
   for (auto &a : atoms) S += a.nrad;
@@ -752,21 +750,16 @@ void DeviceGrid::exchange_potential(int ndim, const double *d_psi, const double 
   xUdt.resize((size_t)nb * S * L);
   if (prof_on) ++prof_calls;
   launch_exchange_chi(d_psi, d_D, ndim, N, xchi.get(), stream);
-  launch_axpby(0.0, xchi.get(), 0.0, xchi.get(), (long)ndim * N, d_K, stream);  // K = 0
-  for (int c0 = 0; c0 < npair; c0 += SET_BATCH) {
-    const int cnt = std::min(SET_BATCH, npair - c0);
+  for (long c0 = 0; c0 < npair; c0 += SET_BATCH) {
+    const int cnt = (int)std::min<long>(SET_BATCH, npair - c0);
     tic(1);
-    for (int k = 0; k < cnt; ++k)
-      launch_mul(d_psi + (long)prs[c0 + k].first * N, d_psi + (long)prs[c0 + k].second * N, N,
-                 xdens.get() + (long)k * N, stream);
+    launch_exchange_dens(d_psi, c0, cnt, N, xdens.get(), stream);
     launch_project(at, xdens.get(), bw.get(), pl.yhat.get(), lmax, xrho.get(), stream, cnt, N, S * L);
     launch_radial(at, xrho.get(), pl.green.get(), lmax, xUy.get(), xUdt.get(), stream, cnt, S * L);
     toc();
     synth_sets(lmax, cnt, xUy.get(), xUdt.get(), S * L, xaux.get(), N);
     tic(6);
-    for (int k = 0; k < cnt; ++k)
-      launch_exchange_acc(xaux.get() + (long)k * N, xchi.get(), prs[c0 + k].first,
-                          prs[c0 + k].second, N, d_K, stream);
+    launch_exchange_acc(xaux.get(), xchi.get(), ndim, c0, cnt, N, d_K, stream);
     toc();
   }
 }
