@@ -3,6 +3,7 @@
 
 #include <map>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "common.hpp"
@@ -184,6 +185,9 @@ struct DeviceGrid {
   // arrays: K [ndim x N] = sum_k sum_l psi_k V[psi_l psi_j] D[k][l] by ndim(ndim+1)/2
   // Poisson solves of orbital products.
   void exchange_potential(int ndim, const double *d_psi, const double *d_D, int lmax, double *d_K);
+  // Device copies of the host entry points' arrays (HostStage in api.cpp), kept between calls.
+  DeviceBuffer<double> stage;
+  std::mutex stage_mu;
   DeviceBuffer<double> xchi, xdens, xaux;  // its workspace, kept between calls
   DeviceBuffer<double> xrho, xUy, xUdt;    // per batch of orbital pairs
   // Synthesis of nset densities on this grid from their radial solutions (set s at
