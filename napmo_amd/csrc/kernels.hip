@@ -103,90 +103,148 @@ void launch_collocate(const double *x, const double *y, const double *z, long N,
 }
 
 // ========================================================= Poisson: projection
-// rho_lm[A][i][lm] = sum_j f_Aij Yhat[j][lm] with f = dens * bw, as a small GEMM per
-// atom: one workgroup per (atom, block of PSB radial shells) so the Lebedev table
-// Yhat[j][lm] = aw_j S_lm(u_j) sqrt(4 pi (2l+1)) / sum aw is read once per block; the
-// shells' f values are staged in LDS in chunks of PJ angular points.
-constexpr int PSB = 5, PJ = 256;
+// rho_lm[A][i][lm] = sum_j f_Aij Yhat[j][lm] with f = dens * bw and the Lebedev table
+// Yhat[j][lm] = aw_j S_lm(u_j) sqrt(4 pi (2l+1)) / sum aw: per atom a product of nset x nrad
+// rows (density o, shell i) with Yhat, on FP64 MFMA. One workgroup forms 16 R rows x 16 C harmonics;
+// its 8 waves share the angular points in groups of four (wave w the groups w, w + 8, ...), f is
+// staged in LDS PJ points at a time (the next PJ read meanwhile), Yhat goes straight to the
+// operand registers, and the waves' sums are added in order at the end. What bounds the product
+// is reading Yhat from L2, once per 16 R rows (the rows of one density, 5 a workgroup, read
+// 5.8 GB for 40 densities): 16 atoms x 50 x 590 points, lmax 12, 40 densities 0.63 -> 0.22
+// ms, one density 24 -> 21 us; 8 atoms, 21 densities 74 -> 37 us. A row's sum does not depend on
+// R and C, nor on the densities that share the launch.
+constexpr int PJ = 128, PPITCH = PJ + 2, PWAVES = 8;
 
-// Threads: 64 lm x PSL angular slices; slice k sums angular points j = k, k + PSL, ... (two
-// independent loads in flight per step); slices are combined in order through LDS.
-template <int PSL>
-__global__ void __launch_bounds__(64 * PSL) k_project(AtomTables at, const double *__restrict__ dens,
-                                                      const double *__restrict__ bw,
-                                                      const double *__restrict__ yhat, int L,
-                                                      double *__restrict__ rho_lm, long dstride,
-                                                      long ostride) {
-  __shared__ double sf[PSB][PJ];
-  __shared__ double red[PSL][PSB][64];
-  // blockIdx.z = o M + A: density o (dens + o dstride -> rho_lm + o ostride), atom A
-  const int A = blockIdx.z % at.M, o = blockIdx.z / at.M;
-  dens += o * dstride;
-  rho_lm += o * ostride;
-  const int i0 = blockIdx.x * PSB;
-  const int nr = at.nrad[A];
-  if (i0 >= nr) return;
-  const int ns = min(PSB, nr - i0);
-  const int na = at.nang[A];
-  const long p0 = at.point_off[A] + (long)i0 * na;
-  const double *Y = yhat + at.yhat_off[A];
-  const int lml = threadIdx.x & 63, slice = threadIdx.x >> 6;
-  const int lm = blockIdx.y * 64 + lml;
+template <int R, int C>
+__global__ void __launch_bounds__(64 * PWAVES, 4) k_project(AtomTables at, const double *__restrict__ dens,
+                                                         const double *__restrict__ bw,
+                                                         const double *__restrict__ yhat, int L,
+                                                         double *__restrict__ rho_lm, int nset,
+                                                         long dstride, long ostride) {
+  constexpr int ROWS = 16 * R, NV = ROWS * PJ / (64 * PWAVES);
+  constexpr int CP = C > 1 ? 2 : 1, NG = PJ / 4 / PWAVES;
+  __shared__ double sh[ROWS * PPITCH > PWAVES * 256 * CP ? ROWS * PPITCH : PWAVES * 256 * CP];
+  __shared__ long row_d[ROWS], row_p[ROWS], row_o[ROWS];
+  const int A = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int nr = at.nrad[A], na = at.nang[A];
+  const int rows = nset * nr, q0 = blockIdx.x * ROWS, lm0 = blockIdx.y * 16 * C;
+  if (q0 >= rows) return;
+  if (tid < ROWS) {  // rows past the last repeat it and are not written
+    const int q = min(q0 + tid, rows - 1), o = q / nr, i = q % nr;
+    row_p[tid] = at.point_off[A] + (long)i * na;
+    row_d[tid] = o * dstride + row_p[tid];
+    row_o[tid] = o * ostride + (at.rad_off[A] + i) * (long)L;
+  }
+  __syncthreads();
   // harmonics above the centre's cut are zero (written, not summed)
   const int Lc = at.lcut ? (at.lcut[A] + 1) * (at.lcut[A] + 1) : L;
-  double acc[PSB];
+  const int kr = lane >> 4, mi = lane & 15;
+  d4 acc[R][C];
 #pragma unroll
-  for (int k = 0; k < PSB; ++k) acc[k] = 0.0;
-  for (int j0 = 0; j0 < na; j0 += PJ) {
-    const int nj = min(PJ, na - j0);
-    __syncthreads();
-    for (int e = threadIdx.x; e < PSB * PJ; e += blockDim.x) {
-      const int k = e / PJ, j = e % PJ;
-      const long p = p0 + (long)k * na + j0 + j;
-      sf[k][j] = (k < ns && j < nj) ? dens[p] * bw[p] : 0.0;
-    }
-    __syncthreads();
-    if (lm < Lc) {
-      // pairs (j, j + PSL) in order; the Yhat loads of the next two pairs are in flight
-      // while one pair is summed
-      int j = slice;
-      const double *Yc = Y + (long)j0 * L + lm;
-      double ya0 = 0, ya1 = 0, yb0 = 0, yb1 = 0;
-      if (j + PSL < nj) ya0 = Yc[(long)j * L], ya1 = Yc[(long)(j + PSL) * L];
-      if (j + 3 * PSL < nj) yb0 = Yc[(long)(j + 2 * PSL) * L], yb1 = Yc[(long)(j + 3 * PSL) * L];
-      for (; j + PSL < nj; j += 2 * PSL) {
-        const double y0 = ya0, y1 = ya1;
-        ya0 = yb0, ya1 = yb1;
-        if (j + 5 * PSL < nj) yb0 = Yc[(long)(j + 4 * PSL) * L], yb1 = Yc[(long)(j + 5 * PSL) * L];
+  for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int k = 0; k < PSB; ++k) acc[k] += sf[k][j] * y0 + sf[k][j + PSL] * y1;
+    for (int c = 0; c < C; ++c) acc[r][c] = (d4){0, 0, 0, 0};
+  if (lm0 < Lc) {
+    const int sj = tid & (PJ - 1), sr = tid / PJ;
+    double vd[NV], vb[NV];
+    auto load = [&](int j0) {
+      const int j = min(j0 + sj, na - 1);
+#pragma unroll
+      for (int t = 0; t < NV; ++t) {
+        const int row = sr + t * (64 * PWAVES / PJ);
+        vd[t] = dens[row_d[row] + j], vb[t] = bw[row_p[row] + j];
       }
-      for (; j < nj; j += PSL) {
-        const double y = Y[(long)(j0 + j) * L + lm];
+    };
+    const double *Y = yhat + at.yhat_off[A];
+    int col[C];
 #pragma unroll
-        for (int k = 0; k < PSB; ++k) acc[k] += sf[k][j] * y;
+    for (int c = 0; c < C; ++c) col[c] = min(lm0 + 16 * c + mi, L - 1);
+    auto yload = [&](int j0, int u, double *y) {
+      const int off = min(j0 + 4 * (wave + u * PWAVES) + kr, na - 1) * L;
+#pragma unroll
+      for (int c = 0; c < C; ++c) y[c] = Y[(unsigned)(off + col[c])];
+    };
+    auto multiply = [&](int u, const double *b) {
+      double a[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) a[r] = sh[(16 * r + mi) * PPITCH + 4 * (wave + u * PWAVES) + kr];
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+          acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[r], b[c], acc[r][c], 0, 0, 0);
+    };
+    double y[NG][C];
+    load(0);
+    if (C == 1)
+#pragma unroll
+      for (int u = 0; u < NG; ++u) yload(0, u, y[u]);
+    for (int j0 = 0; j0 < na; j0 += PJ) {
+#pragma unroll
+      for (int t = 0; t < NV; ++t)
+        sh[(sr + t * (64 * PWAVES / PJ)) * PPITCH + sj] = j0 + sj < na ? vd[t] * vb[t] : 0.0;
+      __syncthreads();
+      if (j0 + PJ < na) load(j0 + PJ);
+      if (C == 1) {
+        // few products: the wave's whole share of the next PJ points is in flight
+        double b[NG][C];
+#pragma unroll
+        for (int u = 0; u < NG; ++u) b[u][0] = y[u][0];
+#pragma unroll
+        for (int u = 0; u < NG; ++u) yload(j0 + PJ, u, y[u]);
+#pragma unroll
+        for (int u = 0; u < NG; ++u) multiply(u, b[u]);
+      } else {
+        const int ng = ((min(PJ, na - j0) + 3) / 4 - wave + PWAVES - 1) / PWAVES;
+        yload(j0, 0, y[0]);
+        for (int u = 0; u < ng; ++u) {
+          double b[C];
+#pragma unroll
+          for (int c = 0; c < C; ++c) b[c] = y[0][c];
+          yload(j0, u + 1, y[0]);
+          multiply(u, b);
+        }
       }
+      __syncthreads();
     }
   }
+  // the waves' sums, 16 rows x 16 CP harmonics at a time (element e of a lane: row kr + 4 e)
 #pragma unroll
-  for (int k = 0; k < PSB; ++k) red[slice][k][lml] = acc[k];
-  __syncthreads();
-  if (slice == 0 && lm < L)
-    for (int k = 0; k < ns; ++k) {
+  for (int h = 0; h < R * C / CP; ++h) {
+    const int r = h / (C / CP), c0 = h % (C / CP) * CP;
+#pragma unroll
+    for (int c = 0; c < CP; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        sh[(wave * 16 + kr + 4 * e) * 16 * CP + 16 * c + mi] = acc[r][c0 + c][e];
+    __syncthreads();
+    if (tid < 256 * CP) {
       double t = 0.0;
-      for (int sl = 0; sl < PSL; ++sl) t += red[sl][k][lml];
-      rho_lm[(at.rad_off[A] + i0 + k) * (long)L + lm] = lm < Lc ? t : 0.0;
+#pragma unroll
+      for (int w = 0; w < PWAVES; ++w) t += sh[w * 256 * CP + tid];
+      const int row = 16 * r + tid / (16 * CP), lm = lm0 + 16 * c0 + tid % (16 * CP);
+      if (q0 + row < rows && lm < L) rho_lm[row_o[row] + lm] = lm < Lc ? t : 0.0;
     }
+    __syncthreads();
+  }
 }
 
 void launch_project(const AtomTables &at, const double *dens, const double *bw, const double *yhat,
                     int lmax, double *rho_lm, hipStream_t s, int nset, long dstride, long ostride) {
   const int L = (lmax + 1) * (lmax + 1);
   NAPMO_REQUIRE(nset >= 1 && (long)nset * at.M <= 65535, "projection: too many density sets");
-  dim3 grid(div_up(at.max_nrad, PSB), div_up(L, 64), nset * at.M);
-  // one slice count for every batch size, so a density's projections do not depend on
-  // how many densities share the launch
-  k_project<16><<<grid, 64 * 16, 0, s>>>(at, dens, bw, yhat, L, rho_lm, dstride, ostride);
+  const long rows = (long)nset * at.max_nrad, cols = div_up(L, 64) * at.M;
+  auto grid = [&](int r, int c) { return dim3((unsigned)div_up(rows, r), (unsigned)div_up(L, c), at.M); };
+  // 32 rows x 64 harmonics read Yhat and f least, with at least two workgroups a CU (40 densities
+  // on 16 atoms 0.22 ms; at 528 workgroups, 21 densities on 8 atoms, 16 rows take the same 37 us);
+  // 16 rows down to one a CU (24 atoms, one density: 288 workgroups 26 us, 16 x 16 37 us); else
+  // 16 x 16 (16 atoms: 192 workgroups of 16 x 64 21 us, 16 x 16 21 us; 3 atoms 10 -> 7.8 us)
+  if (div_up(rows, 32) * cols >= 512)
+    k_project<2, 4><<<grid(32, 64), 64 * PWAVES, 0, s>>>(at, dens, bw, yhat, L, rho_lm, nset, dstride, ostride);
+  else if (div_up(rows, 16) * cols >= 256)
+    k_project<1, 4><<<grid(16, 64), 64 * PWAVES, 0, s>>>(at, dens, bw, yhat, L, rho_lm, nset, dstride, ostride);
+  else
+    k_project<1, 1><<<grid(16, 16), 64 * PWAVES, 0, s>>>(at, dens, bw, yhat, L, rho_lm, nset, dstride, ostride);
   NAPMO_HIP(hipGetLastError());
 }
 
