@@ -601,8 +601,8 @@ def batch_leg(args, log):
     }
 
 
-PHASE_KERNELS = {'density': 'k_density_mfma',
-                 'fock': {'bf16x3': 'k_fock_bf16x3_pass', 'fp64': 'k_fock_f64', 'int8': 'k_ozaki_fock',
+PHASE_KERNELS = {'density': 'k_density_tiles',
+                 'fock': {'bf16x3': 'k_fock_bf16x3_pass', 'fp64': 'k_fock_blocks', 'int8': 'k_ozaki_fock',
                           'int8s': 'k_ozaki_fock'},
                  'synth': 'k_synth2n<', 'project': 'k_project', 'radial': 'k_radial',
                  'fock_reduce': 'k_fock_reduce'}
@@ -644,7 +644,7 @@ def measured_traffic(res, phase):
     if phase == 'density':
         # orbital form: the streamed kernel (C resident in LDS) when the profile has it
         stream = [k for k in kern if 'k_density_orb_stream' in k]
-        tag = ', 1, ' if res['form'] == 'C' else ', 0, '
+        tag = ', false>' if res['form'] == 'C' else ', true>'
         names = (stream if res['form'] == 'C' and stream else
                  [k for k in names if tag in k] or names)
     for k in names:
