@@ -32,7 +32,7 @@ struct FockPlan {
   DeviceBuffer<float> phiT32;          // function-major [ld x Npad]
   DeviceBuffer<double> Cpad, Pfull;    // orbital-form inputs
   DeviceBuffer<double> P, rho_part, rho, v, s, F_part, F, E, trace_work;
-  FockShape fsh, psh;  // per-tile shape; one-pass shape (mixed mode)
+  FockShape fsh, psh;  // per-tile shape (overlap, mixed mode); one-pass shape (mixed mode)
   FockShape dsh;       // FP64 contraction: upper blocks, or fsh past FOCK_MAX_NB block rows
   // int8 mode: digit planes of sqrt|w bw| Phi, chunk exponents, per-stage max |d1|, the
   // per-build signed potential vs = sign(w bw) v, partials, wave tasks (+ group rows)
