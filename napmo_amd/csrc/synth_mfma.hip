@@ -18,6 +18,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "synth_rows.hpp"
 
 namespace napmo {
 
@@ -70,27 +71,26 @@ __device__ __forceinline__ void smf_body(const double (&g0)[4], const double (&u
   }
   // coefficients of the next SMF_PD steps: rows q (cos) and q + 1 (sin; not used for m = 0),
   // through a buffer descriptor of the bucket's rows: lane offset + scalar offset, no address
-  // arithmetic on the VALU; rows past the end read as zero
+  // arithmetic on the VALU. Past the last step the last row is read again, and its features are
+  // zero.
   const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)row, 0, (int)(L * qstride * 8), 0x00020000);
-  const int qbytes = (int)qstride * 8;
+  const int qbytes = (int)qstride * 8, qlast = (L - 1) * qbytes;
   double rt[SMF_PD][2][TW > 0 ? TW : 1], rq[SMF_PD][2][T4 > 0 ? T4 : 1];
-  int ql = 0, ll = 0, ml = 0;  // the load stream's row offset, l, m
+  SynthRows next;  // of the load stream
   auto fetch = [&](unsigned v, int so) {
     const smf_u2 r = __builtin_amdgcn_raw_buffer_load_b64(rsrc, (int)v, so, 0);
     return __builtin_bit_cast(double, r);
   };
   auto load = [&](int k) {
+    const int so[2] = {next.cos_row(qlast), next.sin_row(qbytes, qlast)};
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
 #pragma unroll
-      for (int t = 0; t < TW; ++t) rt[k][h][t] = fetch(tofs + t * tstep, ql + h * qbytes);
+      for (int t = 0; t < TW; ++t) rt[k][h][t] = fetch(tofs + t * tstep, so[h]);
 #pragma unroll
-      for (int t = 0; t < T4; ++t) rq[k][h][t] = fetch(qofs + t * qstep, ql + h * qbytes);
+      for (int t = 0; t < T4; ++t) rq[k][h][t] = fetch(qofs + t * qstep, so[h]);
     }
-    ql += ml ? 2 * qbytes : qbytes;
-    const bool end = ll == lmax;
-    ml += end ? 1 : 0;
-    ll = end ? ml : ll + 1;
+    next.next(lmax, qbytes);
   };
   auto products = [&](const double (&f)[4], const double (&ct)[TW > 0 ? TW : 1], const double (&cq)[T4 > 0 ? T4 : 1]) {
 #pragma unroll
@@ -109,7 +109,7 @@ __device__ __forceinline__ void smf_body(const double (&g0)[4], const double (&u
   int l = 0, m = 0;
   double beta = 0.0;  // of the next l, read one step ahead
   // whole groups of SMF_PD steps (no early exit, so that the waits keep the loads in flight):
-  // past the last step the features and the coefficient rows are zero
+  // past the last step the features are zero
 #pragma unroll 1
   for (int s = 0; s < steps; s += SMF_PD) {
 #pragma unroll
