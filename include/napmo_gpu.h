@@ -454,7 +454,8 @@ enum {
   NAPMO_TUNE_BACKWARD_POINTS = 10, /* energy derivatives (dE/dP, dE/dR): 0 = from the stored
                                      Phi with Phi P for all points at once; k > 0 = Phi
                                      recollocated in chunks of about k points (rounded up to
-                                     a multiple of the contraction chunks), neither the stored
+                                     whole chunks of the derivative's own reduction; read back:
+                                     the points that the chunk buffers hold), neither the stored
                                      Phi nor a full Phi P read: the same results bit for bit */
   NAPMO_TUNE_INT8_SCREEN = 11, /* int8 mode: S > 0 skips, per chunk of points, the 16 x 16 blocks
                                  of F whose chunk sum is bounded by 2^-S in every element (from

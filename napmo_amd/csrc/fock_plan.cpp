@@ -456,13 +456,13 @@ void FockPlan::symmetric_weight() {
   launch_half_sum(s.get(), adj_z.get(), grid.N, Npad, ssym.get(), st);
 }
 
-// Points per chunk of the recollocating backward: a multiple of the Fock chunk, of the
-// gradient's 4096-point chunk and of the density tile, so every partial sum covers the same
-// points as in the stored-Phi path.
-long FockPlan::backward_chunk() const {
-  const long unit = std::lcm(std::lcm(dsh.chunk, grad_chunk_points()), 256L);
-  return std::max<long>(1, div_up(std::max<long>(bwd_points, 1), unit)) * unit;
-}
+// Points per chunk of the recollocating backward. Each derivative takes whole chunks of its own
+// reduction, so that every partial sum covers the same points as in the stored-Phi path: dE/dP
+// chunks of the contraction, dE/dR the 4096-point chunks of the gradient (a common multiple of
+// both can be the whole grid: 3712 and 4096 points meet at 118,784).
+long FockPlan::backward_chunk_dP() const { return round_up(std::max<long>(bwd_points, 1), std::lcm(dsh.chunk, 64L)); }
+long FockPlan::backward_chunk_dR() const { return round_up(std::max<long>(bwd_points, 1), std::lcm(grad_chunk_points(), 256L)); }
+long FockPlan::backward_chunk() const { return std::max(backward_chunk_dP(), backward_chunk_dR()); }
 
 void FockPlan::energy_dP(double *dEdP) {
   symmetric_weight();
@@ -472,8 +472,8 @@ void FockPlan::energy_dP(double *dEdP) {
   } else {
     // Phi recollocated chunk by chunk; each chunk's Fock partials land where the stored-Phi
     // launch writes them
-    const long C = backward_chunk();
-    bwd_phi.resize((size_t)std::min(C, Npad) * ld);
+    const long C = backward_chunk_dP();
+    bwd_phi.resize((size_t)std::min(backward_chunk(), Npad) * ld);
     for (long p0 = 0; p0 < Npad; p0 += C) {
       const long cn = std::max<long>(0, std::min(C, grid.N - p0)), cpad = std::min(C, Npad - p0);
       basis.collocate(grid.x.get() + p0, grid.y.get() + p0, grid.z.get() + p0, cn, cpad, ld,
@@ -505,8 +505,8 @@ void FockPlan::gradient_device(const double *dP, double *dG) {
   }
   // Phi recollocated and Phi P formed chunk by chunk; the partial sums of every 4096-point
   // chunk land where the one-pass kernel writes them, then one reduction
-  const long C = backward_chunk();
-  bwd_phi.resize((size_t)std::min(C, Npad) * ld);
+  const long C = backward_chunk_dR();
+  bwd_phi.resize((size_t)std::min(backward_chunk(), Npad) * ld);
   bwd_X.resize((size_t)std::min(C, Npad) * ld);
   for (long p0 = 0; p0 < grid.N; p0 += C) {
     const long cn = std::min(C, grid.N - p0), cpad = std::min(C, Npad - p0);

@@ -121,7 +121,9 @@ struct FockPlan {
   // NAPMO_TUNE_BACKWARD_POINTS: 0, or the points per chunk of recollocated Phi
   long bwd_points = 0;
   DeviceBuffer<double> bwd_phi, bwd_X;
-  long backward_chunk() const;
+  long backward_chunk_dP() const;  // for dE/dP
+  long backward_chunk_dR() const;  // for dE/dR
+  long backward_chunk() const;     // the larger: what the buffers hold
   void adjoint_potential(const double *y, double *z);
   void symmetric_weight();
   void energy_dP(double *dEdP);

@@ -201,3 +201,30 @@ def test_recollocating_backward_matches_stored_phi(case):
               % (case, v.value, pts, g.size, np.array_equal(dP1, dP0), np.array_equal(gR1, gR0)))
         assert np.array_equal(dP1, dP0) and np.array_equal(gR1, gR0)
     cext.check(cext.napmo_fock_plan_set_tuning(f._this, key, 0))
+
+
+@pytest.mark.parametrize('natom, nrad, nang, ncycle', [(16, 50, 590, 30), (24, 75, 590, 48)])
+def test_recollocating_backward_keeps_its_chunk_small(natom, nrad, nang, ncycle):
+    # The key exists to bound memory: the least chunk is one chunk of each derivative's own
+    # reduction, 4,096 points for dE/dR and for dE/dP one contraction chunk (at most 1 / 64 of the
+    # grid, for a device of 256 workgroups in 4 strips, rounded up to 64 points), however the two
+    # divide each other; and the results stay those of the stored Phi, bit for bit.
+    import ctypes
+    import napmo_amd
+    from napmo_amd import workloads
+    from napmo_amd.system import cext
+    atoms, shells, _, _, _ = workloads.chon16_system(natom=natom, ncycle=ncycle)
+    g, b = systems.gpu_system(atoms, shells, None, None, sizes=[(nrad, nang)] * natom)
+    f = napmo_amd.GridFock(g, b, 2, 'fp64')
+    P = np.random.default_rng(natom).normal(size=(f.nbasis, f.nbasis))
+    P = 0.01 * (P + P.T)
+    f.build(P)
+    dP0, gR0 = f.energy_dP(), f.gradient(P)
+    key, v = 10, ctypes.c_long()
+    for pts in (1, 20000):
+        cext.check(cext.napmo_fock_plan_set_tuning(f._this, key, pts))
+        cext.check(cext.napmo_fock_plan_get_tuning(f._this, key, ctypes.byref(v)))
+        print('%d functions, %d points: %d points asked, %d taken' % (f.nbasis, g.size, pts, v.value))
+        assert pts <= v.value < pts + max(4096, g.size // 64 + 128)
+        assert np.array_equal(f.energy_dP(), dP0) and np.array_equal(f.gradient(P), gR0)
+    cext.check(cext.napmo_fock_plan_set_tuning(f._this, key, 0))
