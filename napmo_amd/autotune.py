@@ -1,13 +1,13 @@
 """Launch-shape autotuner for grid Fock plans.
 
 For a plan (one molecule's grid, basis and precision) it times every candidate launch
-shape of the Fock contraction on the device (the per-tile FP64 / BF16x3 kernels' workgroup
+shape of the Fock contraction on the device (the FP64 and per-tile BF16x3 kernels' workgroup
 count, the one-pass BF16x3 kernel's workgroup count, and the choice between the two
 BF16x3 kernels), then the synthesis' pairs per lane (1 or 2) together with the orbital-form density's
 choice of kernel (C resident in LDS with Phi streamed in one of two launch shapes, or the
-LDS-staged kernel), keeps the fastest, and stores it in a JSON cache keyed by the shape class
-(precision, padded basis size, point count rounded to a power of two), so later plans of
-the same class start from the cached choice without timing. The cache lives at
+column-tile kernel), keeps the fastest, and stores it in a JSON cache keyed by the shape class
+(precision, padded basis size, point count rounded to a power of two) and the generation of the
+kernels, so later plans of the same class start from the cached choice without timing. The cache lives at
 $NAPMO_TUNING_CACHE or ~/.cache/napmo_amd/tuning.json.
 """
 import ctypes
@@ -26,8 +26,10 @@ _KEYS = {'fock_wg': TUNE_FOCK_WG, 'pass_wg': TUNE_PASS_WG, 'use_pass': TUNE_USE_
          'density_stream': TUNE_DENSITY_STREAM, 'int8_chunk': TUNE_INT8_CHUNK,
          'int8_wave_blocks': TUNE_INT8_WAVE_BLOCKS, 'int8_pack': TUNE_INT8_PACK}
 _INT8_KEYS = ('int8_chunk', 'int8_wave_blocks', 'int8_pack')   # only int8 plans have them
-DEFAULTS = {'fock_wg': 0, 'pass_wg': 0, 'density_ks': 16, 'density_pf': 1,
-            'synth_np': 2, 'density_stream': 1}   # 0: the library's default shape
+DEFAULTS = {'fock_wg': 0, 'pass_wg': 0, 'synth_np': 2, 'density_stream': 1}   # 0: the library's default shape
+# Part of the cache key, raised when a kernel that these settings launch is replaced: a choice
+# timed on the old one says nothing about the new one.
+KERNELS = 2
 
 
 def cache_path():
@@ -38,7 +40,7 @@ def cache_path():
 def shape_key(fock):
     ld = -(-fock.nbasis // 64) * 64
     nb = 1 << max(0, int(round(math.log2(max(fock.npoint, 1)))))
-    return '%s:ld%d:N%d' % (fock.precision, ld, nb)
+    return '%s:ld%d:N%d:k%d' % (fock.precision, ld, nb, KERNELS)
 
 
 def candidates(fock):
@@ -58,8 +60,15 @@ def candidates(fock):
         # the symmetric form only with short chunks (its FP32 chunk sums drift otherwise)
         out += [{'use_pass': 2, 'pass_wg': w} for w in (1024, 2048)]
         out += [{'use_pass': 0, 'fock_wg': w} for w in (1024, 2048, 4096)]
+    elif fock.nbasis <= 640:
+        # upper 16 x 16 blocks. The default (0) is one round of the workgroups that the device
+        # holds (256 from 161 functions on, 512 or 768 below) and mostly the fastest: contraction
+        # and reduction at 300 functions x 472,000 points 754 us, two rounds 769, four 801, 16
+        # 1024 us. Around 130 functions half a round leaves fewer partials (82.6 against 86.6 us).
+        # Every chunk of points is a whole partial of F, so more rounds than four only cost memory.
+        out = [{'fock_wg': w} for w in (0, 256, 512, 1024)]
     else:
-        out = [{'fock_wg': w} for w in (512, 1024, 2048, 4096, 8192)]
+        out = [{'fock_wg': w} for w in (0, 512, 1024, 4096, 8192)]
     return out
 
 
