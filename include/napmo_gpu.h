@@ -448,9 +448,9 @@ enum {
   NAPMO_TUNE_SYNTH_MFMA_MIN = 9, /* many-density synthesis (exchange potential, orbital
                                    corrections): whole tiles of 16 densities, and a last tile
                                    of at least this many (in fours), run on FP64 MFMA, the
-                                   others one at a time; 1..16, 17 = one at a time only; 0 = 10,
-                                   the default: by what the last tile costs either way (a
-                                   property of the grid) */
+                                   others one at a time; 1..16, 17 = one at a time only; 0, the
+                                   default = by what the last tile costs either way (reads as
+                                   10; a property of the grid) */
   NAPMO_TUNE_BACKWARD_POINTS = 10, /* energy derivatives (dE/dP, dE/dR): 0 = from the stored
                                      Phi with Phi P for all points at once; k > 0 = Phi
                                      recollocated in chunks of about k points (rounded up to

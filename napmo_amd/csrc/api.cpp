@@ -1075,7 +1075,7 @@ int napmo_grid_set_tuning(void *grid, int key, long value) {
       g.synth_np = value ? (int)value : 2;
     } else if (key == NAPMO_TUNE_SYNTH_MFMA_MIN) {
       NAPMO_REQUIRE(value >= 0 && value <= 17, "MFMA synthesis threshold must be 0 to 17");
-      g.synth_mfma_min = value ? (int)value : SYNTH_MFMA_MIN;
+      g.synth_mfma_min = (int)value;
     } else {
       throw Error("unknown grid tuning key " + std::to_string(key));
     }
@@ -1087,7 +1087,7 @@ int napmo_grid_get_tuning(void *grid, int key, long *value) {
     if (key == NAPMO_TUNE_SYNTH_NP)
       *value = g.synth_np;
     else if (key == NAPMO_TUNE_SYNTH_MFMA_MIN)
-      *value = g.synth_mfma_min;
+      *value = g.synth_mfma_min ? g.synth_mfma_min : SYNTH_MFMA_MIN;
     else
       throw Error("unknown grid tuning key " + std::to_string(key));
   });

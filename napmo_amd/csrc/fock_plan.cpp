@@ -111,7 +111,7 @@ void FockPlan::set_tuning(int key, long value) {
       break;
     case NAPMO_TUNE_SYNTH_MFMA_MIN:
       NAPMO_REQUIRE(value >= 0 && value <= 17, "MFMA synthesis threshold must be 0 to 17");
-      grid.synth_mfma_min = value ? (int)value : SYNTH_MFMA_MIN;
+      grid.synth_mfma_min = (int)value;
       break;
     case NAPMO_TUNE_BACKWARD_POINTS: bwd_points = value; break;
     case NAPMO_TUNE_DENSITY_STREAM:
@@ -167,7 +167,7 @@ long FockPlan::get_tuning(int key) const {
     case NAPMO_TUNE_DENSITY_KS: return density_ks;
     case NAPMO_TUNE_DENSITY_PF: return density_pf;
     case NAPMO_TUNE_SYNTH_NP: return grid.synth_np;
-    case NAPMO_TUNE_SYNTH_MFMA_MIN: return grid.synth_mfma_min;
+    case NAPMO_TUNE_SYNTH_MFMA_MIN: return grid.synth_mfma_min ? grid.synth_mfma_min : SYNTH_MFMA_MIN;
     case NAPMO_TUNE_BACKWARD_POINTS: return bwd_points ? backward_chunk() : 0;
     case NAPMO_TUNE_DENSITY_STREAM: return density_stream;
     case NAPMO_TUNE_DENSITY_SCREEN: return density_screen;

@@ -776,7 +776,7 @@ template <class T> static void grow(DeviceBuffer<T> &b, size_t n) {
 int synth_mfma_count(int nset, int min_tile) {
   if (min_tile > 16) return 0;
   const int rest = nset % 16, full = nset - rest, odd = rest % 4;
-  if (min_tile != SYNTH_MFMA_MIN) return rest >= std::max(min_tile, 1) ? nset : full;
+  if (min_tile > 0) return rest >= min_tile ? nset : full;
   if (full == 0) return rest >= 12 ? nset : 0;
   if (rest < 4) return full;
   return odd <= 2 ? nset - odd : nset;

@@ -77,10 +77,10 @@ constexpr int SET_BATCH = 64;
 // MFMA synthesis: at most this many bytes of per-centre tile sums [M][N][16] at once (at
 // least one tile)
 constexpr long SYNTH_MFMA_BUDGET = 4L << 30;
-// NAPMO_TUNE_SYNTH_MFMA_MIN of a grid; the default stands for the rule of synth_mfma_count.
+// What NAPMO_TUNE_SYNTH_MFMA_MIN reads as where it is not set.
 constexpr int SYNTH_MFMA_MIN = 10;
 // How many of nset densities go through the MFMA synthesis: whole tiles of 16, the rest in fours
-// (13 to 15 as a padded tile).
+// (13 to 15 as a padded tile). min_tile: the fewest that a last tile takes, 0 = by what they cost.
 int synth_mfma_count(int nset, int min_tile);
 
 // Per-geometry pair buckets of the bucketed synthesis (see launch_synth2).
@@ -198,7 +198,7 @@ struct DeviceGrid {
   // sums).
   void synth_sets(int lmax, int nset, const double *Uy, const double *Udt, long ustride,
                   double *out, long ostride, double scale = 1.0);
-  int synth_mfma_min = SYNTH_MFMA_MIN;
+  int synth_mfma_min = 0;  // NAPMO_TUNE_SYNTH_MFMA_MIN, 0: not set
   DeviceBuffer<double> mT, maL, maR, mcontrib;  // its workspace (interleaved tables, tiles)
   DeviceBuffer<double> sT, saL, saR;            // tables of the one-at-a-time densities
   // Residual R = T + V - e psi and de = integrate(R psi) of norb orbitals, then their

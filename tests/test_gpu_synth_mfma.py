@@ -134,3 +134,21 @@ def test_tiles_and_fours(norb, lmax):
     scale = np.abs(b).max(axis=1)
     assert np.all(np.abs(a - b).max(axis=1) < 1e-13 * scale)
     assert np.all(np.abs(run() - b).max(axis=1) < 1e-13 * scale)
+
+
+@pytest.mark.parametrize('norb', [9, 10, 11, 26])
+def test_explicit_threshold_of_ten(norb):
+    # 10 set explicitly is the threshold 10: a last tile of ten or more densities is on MFMA (the
+    # bits of threshold 1), nine are not (the bits of 17). Left at 0 the library decides by cost.
+    import napmo_amd
+    g, _ = systems.gpu_system(ATOMS, [[]] * 3, 12, 26)
+    o, _ = systems.oracle_system(ATOMS, [[]] * 3, 12, 26)
+    phi, ri, V = _orbital_inputs(o, norb, 5)
+    doi, oi = np.linspace(0.02, -0.01, norb), np.linspace(-0.6, -0.3, norb)
+    run = lambda: napmo_amd.compute_dpsi(g, 3, phi, doi, oi, ri, V, 1.0)  # noqa: E731
+    a, b = _both(g, run)
+    assert not np.array_equal(a, b)
+    g.set_tuning(MFMA_MIN, 10)
+    assert g.get_tuning(MFMA_MIN) == 10
+    assert np.array_equal(run(), b if norb == 9 else a)
+    g.set_tuning(MFMA_MIN, 0)
