@@ -156,9 +156,8 @@ def test_autotuner_choice_and_cache(tmp_path):
 
 
 def test_every_launch_shape_gives_the_same_build():
-    # all autotuner candidates (Fock workgroup counts, one-pass vs per-tile BF16x3, density
-    # stage depth 16 / 32 and 1 / 2 stages in flight) on one molecule: rho and the energy are
-    # identical to rounding, F within each precision's tolerance
+    # all autotuner candidates (Fock workgroup counts, one-pass vs per-tile BF16x3) on one
+    # molecule: rho and the energy are identical to rounding, F within each precision's tolerance
     from napmo_amd import autotune, workloads
     mols = workloads.batch_molecules(count=1, seed=9)
     for prec in ('fp64', 'bf16x3'):

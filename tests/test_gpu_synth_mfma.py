@@ -152,3 +152,24 @@ def test_explicit_threshold_of_ten(norb):
     assert g.get_tuning(MFMA_MIN) == 10
     assert np.array_equal(run(), b if norb == 9 else a)
     g.set_tuning(MFMA_MIN, 0)
+
+
+@pytest.mark.parametrize('nrad, nang, norb', [(75, 590, 20), (75, 590, 28), (75, 590, 29), (50, 434, 28), (50, 434, 40),
+                                              (50, 434, 44), (50, 434, 45)])
+def test_tiles_within_the_budget(nrad, nang, norb):
+    # 24 centres: at 1,062,000 points a tile of per-centre sums takes 3.3 GB and the 4 GB budget
+    # holds one, at 520,800 points two. One tile: the fours in a launch of their own; two: one tile
+    # and its fours together, two tiles and then fours. Same bound as above.
+    from napmo_amd import workloads
+    from napmo_amd.wavefunction.ndpsi import becke_dickson_step
+    atoms, _, _, _, _ = workloads.chon16_system(natom=24, ncycle=1)
+    g, _ = systems.gpu_system(atoms, [[]] * 24, None, None, sizes=[(nrad, nang)] * 24)
+    r2 = (g.points ** 2).sum(1)
+    psi = np.array([np.exp(-(0.02 + 0.003 * k) * r2) for k in range(norb)])
+    T, V, e = 0.5 * psi, -psi / np.sqrt(r2 + 0.1), np.linspace(-0.6, -0.3, norb)
+    run = lambda: becke_dickson_step(g, 3, psi, T, V, e, 1.0)[0]  # noqa: E731
+    a, b = _both(g, run)
+    scale, err = np.abs(b).max(axis=1), np.abs(a - b).max(axis=1)
+    print('%d orbitals on %d points: max|MFMA - one at a time| %.2e' % (norb, g.size, (err / scale).max()))
+    assert np.all(err < 1e-13 * scale)
+    assert np.all(np.abs(run() - b).max(axis=1) < 1e-13 * scale)
