@@ -605,7 +605,8 @@ PHASE_KERNELS = {'density': 'k_density_tiles',
                  'fock': {'bf16x3': 'k_fock_bf16x3_pass', 'fp64': 'k_fock_blocks', 'int8': 'k_ozaki_fock',
                           'int8s': 'k_ozaki_fock'},
                  'synth': 'k_synth2n<', 'project': 'k_project', 'radial': 'k_radial',
-                 'fock_reduce': 'k_fock_reduce'}
+                 'fock_reduce': {'bf16x3': 'k_fock_reduce<float>', 'fp64': 'k_fock_block_reduce',
+                                 'int8': 'k_ozaki_reduce', 'int8s': 'k_ozaki_reduce'}}
 
 
 def traffic_table(name):

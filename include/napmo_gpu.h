@@ -264,11 +264,15 @@ enum {
   NAPMO_PREC_FP64 = 0,   /* everything float64 (FP64 MFMA) */
   NAPMO_PREC_FP32 = 1,   /* Phi and contractions float32 (FP32 MFMA), FP64 Poisson + traces */
   NAPMO_PREC_BF16X3 = 2, /* 3-term bf16 split on BF16 MFMA, FP32 accumulate, FP64 Poisson */
-  NAPMO_PREC_INT8 = 3    /* F on int8 MFMA: 28-bit digit slices of sqrt|w bw| Phi (per geometry)
+  NAPMO_PREC_INT8 = 3    /* F on int8 MFMA: 35-bit digit slices of sqrt|w bw| Phi (per geometry)
                             and of v times them (per build), exact int32 accumulation per chunk,
                             FP64 across chunks; rho, Poisson and traces FP64 */
 };
 
+/* The calls below that take host arrays stage them on the device: napmo_compute_coulomb,
+ * _kinetic, _exchange_potential, _dpsi and napmo_becke_dickson_step in one buffer that the grid
+ * keeps from call to call (as large as the largest of them, up to 256 MB per grid, freed with
+ * the grid); larger ones allocate for the call. */
 /* Poisson: dens [N] (grid order) -> potential v [N] (napmo/wavefunction/ntwobody.py:15-46). */
 int napmo_compute_coulomb(void *grid, const double *dens, int lmax, double *v_out);
 /* Poisson, expansion only (napmo/grids/poisson_solver.py:18-118): for every centre A and
@@ -311,7 +315,7 @@ int napmo_compute_nuclear(void *grid, int ncharge, const double *charges, const 
  * [norb x N]. Per atom and (l, m) it solves u'' + (2/r) u' + a u = -2/m_inv mu_lm with
  * a = -2/m_inv (l(l+1)/r^2 + V_sph - oi - doi), u = 0 at both radial ends, mu the spherical
  * expansion of (phi doi - ri) bw and V_sph the spherical average of V_tot bw; the solutions
- * are synthesised at every point. Radial grids of 3 to 240 points. */
+ * are synthesised at every point. Radial grids of 3 to 512 points. */
 int napmo_compute_dpsi(void *grid, int lmax, int norb, const double *phi, const double *doi,
                        const double *oi, const double *ri, const double *V_tot, double mass_inv,
                        double *dpsi_out);
@@ -430,7 +434,9 @@ int napmo_grid_poisson_adjoint(void *plan, const double *y, double *z_out);
 /* Launch-shape knobs of a plan, for the autotuner (no reference counterpart). Set them
  * before a batch is captured; not while a build is running. */
 enum {
-  NAPMO_TUNE_FOCK_WG = 0,  /* workgroups of the per-tile Fock kernels (chunks x tiles); 0 = default */
+  NAPMO_TUNE_FOCK_WG = 0,  /* workgroups of the FP64 contraction (chunks x strips of 16 x 16
+                              blocks; x 64 x 64 tiles past 640 functions) and of the per-tile
+                              BF16x3 one (chunks x tiles); every chunk keeps a partial F; 0 = default */
   NAPMO_TUNE_PASS_WG = 1,  /* workgroups of the one-pass BF16x3 Fock kernel; 0 = default */
   NAPMO_TUNE_USE_PASS = 2, /* 0: per-tile BF16x3 kernel, 1: one-pass BF16x3 kernel,
                               2: one-pass kernel on G = sqrt|s| Phi (F = G^T diag(sign s) G) */
@@ -438,9 +444,9 @@ enum {
   NAPMO_TUNE_DENSITY_PF = 4, /* 1 or 2, 0 = 1: accepted and kept, no kernel uses it now */
   NAPMO_TUNE_SYNTH_NP = 5,   /* (point, centre) pairs per lane of the synthesis, 1 or 2; 0 = 2
                                 (a property of the grid: shared by every plan on it) */
-  NAPMO_TUNE_DENSITY_STREAM = 6, /* orbital-form density: 1..4 keep C in LDS and stream Phi when
+  NAPMO_TUNE_DENSITY_STREAM = 6, /* orbital-form density: 1..3 keep C in LDS and stream Phi when
                                    C fits (nocc <= 64), in one of three launch shapes (1: default);
-                                   0 uses the LDS-staged kernels */
+                                   0 uses the column-tile kernel */
   NAPMO_TUNE_INT8_CHUNK = 7,  /* int8 mode: points per chunk (a multiple of 64, at most 4032;
                                  0 = about N / 256). Setting it re-slices the per-geometry digits */
   NAPMO_TUNE_INT8_WAVE_BLOCKS = 8, /* int8 mode: 16 x 16 blocks of F per wave in the row-group

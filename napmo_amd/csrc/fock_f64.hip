@@ -533,9 +533,12 @@ FockShape fock_block_shape(int n, int ld, long Npad, long wg_target) {
   const int nw = nw_of(cw_of(nb));
   sh.nstrip = (int)div_up(T, FOCK_BPW * nw);
   sh.bpw = (int)div_up(div_up(T, sh.nstrip), nw / sh.nset);
-  // one round of the workgroups that the device holds at once, every one the same work (two or
-  // three rounds were no faster and leave more partials to add); at least 128 points each, so
-  // that short grids do not leave mostly partials. Whole pairs of stages: 32 or 64 points.
+  // one round of the workgroups that the device holds at once, every one the same work, since
+  // every further round leaves more partials to add: contraction + reduction at n = 300, 472,000
+  // points in one, two, four rounds 741 + 13, 748 + 21, 763 + 37 us; n = 480, 1,062,000 points
+  // 4112 + 15, 4119 + 25, 4135 + 49; n = 130, 135,900 points in half a round, one, two 72 + 10,
+  // 74 + 13, 82 + 20. At least 128 points each, so that short grids do not leave mostly partials.
+  // Whole pairs of stages: 32 or 64 points.
   const long want = std::max(1L, (wg_target > 0 ? wg_target : (long)FOCK_CUS * occ_of(cw_of(nb))) / sh.nstrip);
   const long per = div_up(Npad, want);
   sh.chunk = std::max(128L, round_up(per, nb <= 3 || per > 1024 ? 64 : 32));

@@ -57,7 +57,7 @@ struct FockPlan {
   int density_ks = 16;            // NAPMO_TUNE_DENSITY_KS: kept, unused
   int density_pf = 1;             // NAPMO_TUNE_DENSITY_PF: kept, unused
   int density_stream = 1;  // orbital form: C resident in LDS, Phi streamed (when it fits), in
-                           // launch shape 1..3; 0: the LDS-staged kernels
+                           // launch shape 1..3; 0: the column-tile kernel
   int density_screen = 0;  // NAPMO_TUNE_DENSITY_SCREEN (0: off)
   DeviceBuffer<double> phi_scr;        // Phi with its columns in the order dens_perm
   DeviceBuffer<int> dens_perm;         // [ld]

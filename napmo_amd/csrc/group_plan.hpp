@@ -37,7 +37,7 @@ struct GroupPlan {
   DeviceBuffer<ScaleMember> smem;
   long dens_blocks = 0, rho_blocks = 0, scale_blocks = 0;
   // Fock contraction: one launch for the members with 4 waves per workgroup, one for those
-  // with 8 (more than 320 functions)
+  // with 8 (161 to 640 functions)
   struct FockGroup {
     DeviceBuffer<FockMember> mem;
     int count = 0;
