@@ -200,3 +200,21 @@ def test_one_launch_per_phase_single_molecule_and_repeated_pointers():
         batch.synchronize()
         assert np.array_equal(dF2[0].to_host(), F), k
         del batch
+
+
+def test_one_launch_per_phase_over_all_contraction_classes():
+    # members of one launch on every class of the FP64 contraction: sets of waves (20 functions),
+    # 4 waves (150), 8 waves (200, 330) and 64 x 64 tiles (660): each equals its own build bit for bit
+    import napmo_amd
+    from tests.test_gpu_fock_blocks import ATOMS, _s_shells
+    sizes = [(30, 50), (22, 110), (17, 26)]
+    mols = [{'atoms': ATOMS, 'shells': _s_shells(n), 'sizes': sizes, 'lmax': 4, 'nocc': 3} for n in (660, 20, 200, 150, 330)]
+    grids, bases, plans, Ps = _setup(mols)
+    dP, dF, dE = _device(Ps)
+    batch = napmo_amd.BatchFock(plans, nlanes=0)
+    batch.build([a.ptr for a in dP], [a.ptr for a in dF], [a.ptr for a in dE])
+    batch.synchronize()
+    for k, (f, P) in enumerate(zip(plans, Ps)):
+        F, E, Eg = f.build(P)
+        Eb = dE[k].to_host()
+        assert np.array_equal(dF[k].to_host(), F) and Eb[0] == E and Eb[1] == Eg, k
