@@ -15,8 +15,8 @@
 // costs 6 to 8 cycles of matrix time (measured), so the product loop holds no other arithmetic:
 // fragment addresses stay in registers and s is multiplied in while staging. What is left above
 // the MFMA time is that staging (LDS writes 15 %, loads 10 % at n = 300).
-// Measured, 64 x 64 tiles -> this: n = 300, 472,000 points 1.02 -> 0.83 ms (55 TFLOP/s on the
-// upper blocks); n = 480, 1,062,000 points 5.4 -> 4.06 ms (62); n = 130, 140,000 points 0.122 ->
+// Measured, 64 x 64 tiles -> this: n = 300, 472,000 points 1.02 -> 0.74 ms (62 TFLOP/s on the
+// upper blocks); n = 480, 1,062,000 points 5.4 -> 4.1 ms (62); n = 130, 140,000 points 0.122 ->
 // 0.086 ms; n = 10, 22,000 points 16.7 -> 6.2 us.
 #include <algorithm>
 
@@ -284,7 +284,7 @@ __host__ __device__ inline int tri_row(int b, int nb) {
 // Shape classes by CW, the LDS row stride of the columns in blocks (odd, so that it is 16 mod
 // 32 doubles): nb = 1, <= 3, 4, <= 8, <= 10, <= 20, <= FOCK_MAX_NB. Short strips use few waves per
 // workgroup and several workgroups per CU; from 11 block rows on 8 waves share a stage, so its
-// columns are staged for twice the blocks (n = 300: 0.86 -> 0.83 ms, n = 480: 4.95 -> 4.06 ms).
+// columns are staged for twice the blocks (4 waves -> 8 on one card: n = 300 0.86 -> 0.83 ms, n = 480 4.95 -> 4.06 ms).
 __host__ __device__ constexpr int cw_of(int nb) {
   return nb == 1 ? 1 : (nb <= 3 ? 3 : (nb == 4 ? 5 : (nb <= 8 ? 9 : (nb <= 10 ? 21 : (nb <= 20 ? 25 : 41)))));
 }
